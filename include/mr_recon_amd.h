@@ -108,8 +108,8 @@ int mra_geom_set_dcf_plan_order(void* geom_host, int on);
  * problem's sample vectors is its s-th sorted sample (no perm gather or scatter). Used by
  * density_compensation (algs.py:20-106), whose iteration never needs sample order. */
 int mra_geom_set_ksp_plan_order(void* geom_host, int on);
-/* Selects the phase-1 kernel behind mra_grid_partial: 1 (default) = 3D cells of samples
- * summed on the matrix cores (P <= 7), 0 = per-lane LDS read-modify-write. Same scratch
+/* Selects the phase-1 kernel behind mra_grid_partial: 1 (default) = samples summed on the
+ * matrix cores (2D, P <= 8; 3D, P <= 7), 0 = per-lane LDS read-modify-write. Same scratch
  * output; returns the previous selection. No reference counterpart (one kernel per
  * dimensionality in grid.py:150-502). */
 int mra_set_grid_kernel(int mode);

@@ -31,6 +31,7 @@
 
 #include "common.h"
 #include "capi_util.h"
+#include "grid_mfma.h"
 
 namespace mra {
 
@@ -802,12 +803,6 @@ __global__ __launch_bounds__(64) void grid_partial_kernel(const float2* __restri
                                                       lds2, rec, wl, vst);
 }
 
-}  // namespace mra
-
-#include "grid_mfma.h"
-
-namespace mra {
-
 // Gridding phase 2. One block per (problem, output tile, group of RB batch entries):
 // sums, in a fixed order, the scratch subgrids of every item whose subgrid covers the
 // tile and writes each grid point once. blockIdx.x = (prob - prob0) * ntiles + tile,
@@ -1435,7 +1430,7 @@ struct LaunchArgs {
 };
 
 
-// Phase-1 gridding kernel: 1 = matrix cores (3D, P <= 7), 0 = per-lane LDS read-modify-write.
+// Phase-1 gridding kernel: 1 = matrix cores (2D, P <= 8; 3D, P <= 7), 0 = per-lane LDS read-modify-write.
 static int g_grid_kernel = 1;
 // Interpolation reads coil pairs as 128-bit LDS values when the coil chunk is even.
 #ifndef MRA_INTERP_PAIRS
@@ -1469,23 +1464,11 @@ static int launch_op(const LaunchArgs& a) {
     }
     case Op::GridPartial: {
       if (a.nitems <= 0) break;
-      if constexpr (D == 3 && P >= 2 && P <= 7) {
-        if (g_grid_kernel == 1) {
-          // A batch that fits one wave's coils runs one wave per block: a second wave
-          // would have no coils but hold half the block's LDS, halving residency.
-          if (a.nbatch <= MfmaGrid<P, 1>::NC) {
-            grid_mfma_kernel<P, 1><<<item_grid(a.nitems, 1), 64, 0, a.stream>>>(
-                (const float2*)a.src, (const float*)a.aux, a.wsort, a.lbase, a.perm, a.geoms, a.items, a.nitems, 1,
-                (float2*)a.dst);
-            break;
-          }
-          using M = MfmaGrid<P>;
-          const int ng = (a.nbatch + M::NC - 1) / M::NC;
-          grid_mfma_kernel<P, M::NW><<<item_grid(a.nitems, ng), 64 * M::NW, 0, a.stream>>>(
-              (const float2*)a.src, (const float*)a.aux, a.wsort, a.lbase, a.perm, a.geoms, a.items, a.nitems, ng,
-              (float2*)a.dst);
-          break;
-        }
+      if (g_grid_kernel == 1 && grid_mfma_supported(D, P)) {
+        launch_grid_mfma(D, P, T,
+                         GridMfmaArgs{(const float2*)a.src, (const float*)a.aux, a.wsort, a.lbase, a.perm, a.geoms,
+                                      a.items, a.nitems, a.nbatch, (float2*)a.dst, a.stream});
+        break;
       }
       using RL = RowLanes<D, P, T>;
       const int nch = (a.nbatch + RL::NC - 1) / RL::NC;
