@@ -48,59 +48,78 @@ __device__ __forceinline__ float2 conjf2(float2 a) { return make_float2(a.x, -a.
 // Forward, last axis: NT pixel rows per block (rows enumerate (q, n0, n1)); grid batch q
 // uses image img_index[q] (or q / ns) and map q (or q % ns).
 template <int L>
-__global__ __launch_bounds__(kThreadsFFT) void pad_row_kernel(const float2* __restrict__ x, long long x_stride,
-                                                               const float2* __restrict__ smaps, long long s_stride,
-                                                               long long ns, const int* __restrict__ img_index,
-                                                               Geo3 p, long long nrows, float2* __restrict__ grid,
-                                                               const float2* __restrict__ twg) {
-  using S = Shape<L, true>;
-  __shared__ float2 buf[L * S::NTP];
-  __shared__ float2 tw[L];
-  // per row of the block: image / map offsets of its pixels, apodization, grid row offset
-  __shared__ long long rsrc[S::NT], rmap[S::NT], rdst[S::NT];
-  __shared__ float rapo[S::NT];
+__global__ __launch_bounds__(Plan<L>::T * Plan<L>::NR) void pad_row_kernel(
+    const float2* __restrict__ x, long long x_stride, const float2* __restrict__ smaps, long long s_stride,
+    long long ns, const int* __restrict__ img_index, Geo3 p, long long nrows, float2* __restrict__ grid,
+    const float2* __restrict__ twg) {
+  using P = Plan<L>;
+  constexpr int NT = P::NR;
+  constexpr bool REV = RowOrder<L>::REV;
+  using TB = Tables<L, REV>;
+  __shared__ float2 buf[BufSize<L, NT>::value];
+  __shared__ float2 tab[TB::SIZE];
+  __shared__ long long rdst[NT];  // grid offset of each row
   const int tid = threadIdx.x;
-  for (int m = tid; m < L; m += kThreadsFFT) tw[m] = twg[m];
-  const long long row0 = (long long)blockIdx.x * S::NT;
+  const int c = tid / P::T, j = tid % P::T;
+  const long long row0 = (long long)blockIdx.x * NT;
   const int N0 = p.N[0], N1 = p.N[1], N2 = p.N[2];
-  if (tid < S::NT) {
-    const long long row = row0 + tid;
-    if (row < nrows) {
-      const int n1 = (int)(row % N1);
-      const long long r2 = row / N1;
-      const int n0 = (int)(r2 % N0);
-      const long long q = r2 / N0;
-      const long long bs = img_index ? q : q % ns;
-      const long long bx = img_index ? img_index[q] : q / ns;
-      const long long pix = ((long long)n0 * N1 + n1) * N2;
-      rsrc[tid] = bx * x_stride + pix;
-      rmap[tid] = bs * s_stride + pix;
-      rapo[tid] = p.scale * apod_at(p, 0, n0) * apod_at(p, 1, n1);
-      rdst[tid] = ((q * p.G[0] + grid_of(n0, p.G[0], p.c[0])) * p.G[1] + grid_of(n1, p.G[1], p.c[1])) * L;
-    }
+  const bool valid = row0 + c < nrows;
+  const float2 *xr = x, *mr = smaps;
+  float a01 = 0.f;
+  if (valid) {
+    const unsigned row = (unsigned)(row0 + c);  // nrows < 2^31
+    const unsigned r2 = row / (unsigned)N1, n1 = row - r2 * N1;
+    const unsigned q = r2 / (unsigned)N0, n0 = r2 - q * N0;
+    const unsigned bq = q / (unsigned)ns;
+    const long long bs = img_index ? q : q - bq * (unsigned)ns;
+    const long long bx = img_index ? img_index[q] : bq;
+    const long long pix = ((long long)n0 * N1 + n1) * N2;
+    xr = x + bx * x_stride + pix;
+    if (smaps) mr = smaps + bs * s_stride + pix;
+    a01 = p.scale * apod_at(p, 0, n0) * apod_at(p, 1, n1);
+    if (j == 0)
+      rdst[c] = (((long long)q * p.G[0] + grid_of(n0, p.G[0], p.c[0])) * p.G[1] + grid_of(n1, p.G[1], p.c[1])) * L;
   }
-  __syncthreads();
-  const int nr = (int)min((long long)S::NT, nrows - row0);
-  for (int e = tid; e < S::NT * L; e += kThreadsFFT) {
-    const int c = e / L, j = e - c * L;
-    float2 v = make_float2(0.f, 0.f);
-    const int n2 = pix_of(j, N2, L, p.c[2]);
-    if (c < nr && n2 >= 0) {
-      v = x[rsrc[c] + n2];
-      if (smaps) v = cmul(v, smaps[rmap[c] + n2]);
-      const float a = rapo[c] * apod_at(p, 2, n2);
-      v.x *= a;
-      v.y *= a;
-    }
-    buf[j * S::NTP + c] = v;
+  // every load first (a grid point without a pixel reads pixel 0), then the products
+  float2 v[TB::A], mv[TB::A], o[TB::Z];
+  float av[TB::A];
+  const bool act = L / TB::A == P::T || j < L / TB::A;
+  auto pix = [&](int q) { return act ? pix_of(j + q * (L / TB::A), N2, L, p.c[2]) : -1; };
+#pragma unroll
+  for (int q = 0; q < TB::A; ++q) v[q] = xr[max(pix(q), 0)];
+  if (smaps) {
+#pragma unroll
+    for (int q = 0; q < TB::A; ++q) mv[q] = mr[max(pix(q), 0)];
   }
-  __syncthreads();
-  fft_lds<L, S>(buf, tw);
-  for (int e = tid; e < S::NT * L; e += kThreadsFFT) {
-    const int c = e / L, j = e - c * L;
-    if (c < nr) grid[rdst[c] + j] = buf[j * S::NTP + c];
+  if (p.apod[2]) {
+#pragma unroll
+    for (int q = 0; q < TB::A; ++q) av[q] = p.apod[2][max(pix(q), 0)];
+  }
+  TB::fill(tab, twg, tid, P::T * NT);
+#pragma unroll
+  for (int q = 0; q < TB::A; ++q) {
+    float2 y = v[q];
+    if (smaps) y = cmul(y, mv[q]);
+    const float a = p.apod[2] ? a01 * av[q] : a01;
+    const bool in = pix(q) >= 0;
+    v[q] = make_float2(in ? y.x * a : 0.f, in ? y.y * a : 0.f);
+  }
+  finish<L, NT, true, REV>(v, o, buf, tab, j, c);
+  if constexpr (RowOrder<L>::STAGE) {
+    stage_rows<L, NT, REV>(o, buf, j, c);
+    for (int e = tid; e < NT * L; e += P::T * NT) {
+      const int r = e / L, i = e - r * L;
+      if (row0 + r < nrows) grid[rdst[r] + i] = buf[Lay<L, TB::A, NT, true>::at(i, r)];
+    }
+  } else {
+    float2* dst = grid + (valid ? rdst[c] : 0);  // written before finish's barrier
+    emit<L, REV>(o, j, [&](int i, int, float2 y) {
+      if (valid) dst[i] = y;
+    });
   }
 }
+
+constexpr unsigned kXCDs = 8;
 
 enum ColMode { kFwd = 0, kAdj = 1, kToep = 2 };
 
@@ -109,149 +128,243 @@ enum ColMode { kFwd = 0, kAdj = 1, kToep = 2 };
 // forward, store all rows. kAdj: load all rows, inverse, store pixel rows. kToep: load
 // pixel rows, forward, multiply by kern (indexed over one grid), inverse, store pixel rows.
 template <int L, int MODE>
-__global__ __launch_bounds__(kThreadsFFT) void col_kernel(float2* __restrict__ grid, Geo3 p, int axis,
-                                                           long long inner, const float2* __restrict__ twg,
-                                                           const float2* __restrict__ kern) {
-  using S = Shape<L, false>;
-  __shared__ float2 buf[L * S::NTP];
-  __shared__ float2 tw[L];
+__global__ __launch_bounds__(Plan<L>::T * Plan<L>::NC) void col_kernel(float2* __restrict__ grid, Geo3 p, int axis,
+                                                                      long long inner, unsigned nblk,
+                                                                      const float2* __restrict__ twg,
+                                                                      const float2* __restrict__ kern) {
+  using P = Plan<L>;
+  constexpr int NT = P::NC;
+  __shared__ float2 buf[BufSize<L, NT>::value];
+  __shared__ float2 tab[Tables<L, false>::SIZE];
   const int tid = threadIdx.x;
-  for (int m = tid; m < L; m += kThreadsFFT) tw[m] = twg[m];
-  const long long nblk = (inner + S::NT - 1) / S::NT;
-  const long long o = blockIdx.x / nblk;
-  const long long i0 = (blockIdx.x - o * nblk) * S::NT;
-  const int nvalid = (int)min((long long)S::NT, inner - i0);
+  const int c = tid % NT, j = tid / NT;
+  // kToep: the outer indices (coils) of a column tile run back to back on one XCD, whose L2
+  // then serves the tile of kern to all but the first (blocks go to the XCDs in turn)
+  unsigned o = blockIdx.x / nblk, t = blockIdx.x - o * nblk;
+  if (MODE == kToep) {
+    const unsigned no = gridDim.x / nblk, l = blockIdx.x / kXCDs, full = nblk / kXCDs * kXCDs;
+    if (blockIdx.x < full * no) {
+      o = l % no;
+      t = l / no * kXCDs + blockIdx.x % kXCDs;
+    } else {
+      const unsigned r = blockIdx.x - full * no;
+      o = r / (nblk - full);
+      t = full + r - o * (nblk - full);
+    }
+  }
+  const long long col0 = (long long)t * NT;
+  const bool valid = col0 + c < inner;
   long long base;
   if (axis == 0) {
-    base = o * (long long)L * inner;
+    base = (long long)o * L * inner;
   } else {  // axis 1: o = q * N0 + n0
-    const long long q = o / p.N[0];
+    const unsigned q = o / (unsigned)p.N[0];
     const int n0 = (int)(o - q * p.N[0]);
-    base = (q * p.G[0] + grid_of(n0, p.G[0], p.c[0])) * (long long)L * inner;
+    base = ((long long)q * p.G[0] + grid_of(n0, p.G[0], p.c[0])) * (long long)L * inner;
   }
   const int Na = p.N[axis], ca = p.c[axis];
-  float2* col = grid + base + i0;
-  for (int e = tid; e < S::NT * L; e += kThreadsFFT) {
-    const int j = e / S::NT, c = e - j * S::NT;
-    float2 v = make_float2(0.f, 0.f);
-    if (c < nvalid) {
-      if (MODE == kAdj) {
-        v = conjf2(col[(long long)j * inner + c]);
-      } else if (pix_of(j, Na, L, ca) >= 0) {
-        v = col[(long long)j * inner + c];
-      }
-    }
-    buf[j * S::NTP + c] = v;
-  }
-  __syncthreads();
-  fft_lds<L, S>(buf, tw);
-  if (MODE == kToep) {
-    const float2* kcol = kern + i0;
-    for (int e = tid; e < S::NT * L; e += kThreadsFFT) {
-      const int j = e / S::NT, c = e - j * S::NT;
-      if (c < nvalid) buf[j * S::NTP + c] = conjf2(cmul(buf[j * S::NTP + c], kcol[(long long)j * inner + c]));
+  const unsigned row = (unsigned)inner * 8u, bytes = L * row;
+  const Slab g(grid + base, bytes);
+  const unsigned off = valid ? j * row + (unsigned)(col0 + c) * 8u : kNone;
+  auto in_pix = [&](int i) { return pix_of(i, Na, L, ca) >= 0; };
+  using TB = Tables<L, false>;
+  float2 v[TB::A], z[TB::Z];
+  load_first<L>(v, j, [&](int i, int d) {
+    const float2 x = g.load(MODE == kAdj || in_pix(i) ? off : kNone, d * row);
+    return MODE == kAdj ? conjf2(x) : x;
+  });
+  if constexpr (MODE == kToep) {
+    using TR = Tables<L, true>;
+    constexpr int NB = L / TR::A;
+    __shared__ float2 tabr[P::R1 == TR::A ? 1 : TR::SIZE];  // equal first and last radix: one table does both
+    const Slab ks(kern, bytes);
+    float2 u[TR::A], y[TR::Z];
+    // loaded with the data; with three passes (1024 threads) that would cost the second block of a CU
+    auto load_kern = [&] { load_first<L>(u, j, [&](int, int d) { return ks.load(off, d * row); }); };
+    if constexpr (!TB::three) load_kern();
+    TB::fill(tab, twg, tid, P::T * NT);
+    if constexpr (P::R1 != TR::A) TR::fill(tabr, twg, tid, P::T * NT);
+    finish<L, NT, false, false>(v, z, buf, tab, j, c);
+    if constexpr (TB::three) load_kern();
+    if (NB == P::T || j < NB) {
+#pragma unroll
+      for (int q = 0; q < TR::A; ++q) u[q] = conjf2(cmul(z[q], u[q]));
     }
     __syncthreads();
-    fft_lds<L, S>(buf, tw);
-  }
-  for (int e = tid; e < S::NT * L; e += kThreadsFFT) {
-    const int j = e / S::NT, c = e - j * S::NT;
-    if (c < nvalid) {
-      if (MODE == kFwd) {
-        col[(long long)j * inner + c] = buf[j * S::NTP + c];
-      } else if (pix_of(j, Na, L, ca) >= 0) {
-        col[(long long)j * inner + c] = conjf2(buf[j * S::NTP + c]);
-      }
-    }
+    finish<L, NT, false, true>(u, y, buf, P::R1 == TR::A ? tab : tabr, j, c);
+    emit<L, true>(y, j, [&](int i, int d, float2 w) { g.store(in_pix(i) ? off : kNone, d * row, conjf2(w)); });
+  } else {
+    TB::fill(tab, twg, tid, P::T * NT);
+    finish<L, NT, false, false>(v, z, buf, tab, j, c);
+    emit<L, false>(z, j, [&](int i, int d, float2 w) {
+      if (MODE == kFwd) g.store(off, d * row, w);
+      else g.store(in_pix(i) ? off : kNone, d * row, conjf2(w));
+    });
   }
 }
 
-constexpr int kCropMaxPix = 3;  // pixels per thread along the last axis (N2 <= 768)
-
-// Adjoint, last axis + crop / coil reduce: one block per image row (bx, n0, n1). Grids
-// [q0, q1) of image bx are inverse-transformed NT at a time and reduced:
-// out[bx][n] (+)= scale * apod(n) * sum_q row_q[g(n)] * (conj) S[q][n].
-template <int L>
-__global__ __launch_bounds__(kThreadsFFT) void crop_row_kernel(const float2* __restrict__ grid, Geo3 p, long long ns,
-                                                                const float2* __restrict__ smaps, long long s_stride,
-                                                                const int* __restrict__ coil_off, int conj_maps,
-                                                                int accumulate, float2* __restrict__ out,
-                                                                long long x_stride, const float2* __restrict__ twg) {
-  using S = Shape<L, true>;
-  __shared__ float2 buf[L * S::NTP];
-  __shared__ float2 tw[L];
+// Adjoint, last axis + crop / coil reduce. A block takes NT / 2^LCB image rows (bx, n0, n1)
+// and 2^LCB coils of each at a time: the grids [q0, q1) of image bx are inverse-transformed
+// and reduced, out[bx][n] (+)= scale * apod(n) * sum_q row_q[g(n)] * (conj) S[q][n]. One coil
+// (LCB = 0) is stored from the registers that end the transform. Otherwise the transforms
+// go back to LDS, where a row's T 2^LCB threads take its pixels, ng threads to a pixel
+// (every ng-th coil each), so that maps are read along the row; the ng partial sums are
+// added at the end, in order.
+template <int L, int LCB>
+__global__ __launch_bounds__(Plan<L>::T * Plan<L>::NA) void crop_row_kernel(
+    const float2* __restrict__ grid, Geo3 p, long long nrows, long long ns, const float2* __restrict__ smaps,
+    long long s_stride, const int* __restrict__ coil_off, int ng, int conj_maps, int accumulate,
+    float2* __restrict__ out, long long x_stride, const float2* __restrict__ twg) {
+  using P = Plan<L>;
+  constexpr int NT = P::NA, CB = 1 << LCB, RB = NT / CB;
+  constexpr bool REV = RowOrder<L>::REV;
+  using TB = Tables<L, REV>;
+  using LY = Lay<L, TB::A, NT, true>;
+  constexpr int GT = P::T * CB;                // threads of an image row
+  constexpr int KM = (L + GT - 1) / GT;        // pixels a thread may own
+  __shared__ float2 buf[BufSize<L, NT>::value];
+  __shared__ float2 tab[TB::SIZE];
   const int tid = threadIdx.x;
-  for (int m = tid; m < L; m += kThreadsFFT) tw[m] = twg[m];
+  const int c = tid / P::T, j = tid % P::T;
   const int N0 = p.N[0], N1 = p.N[1], N2 = p.N[2];
-  const long long row = blockIdx.x;
-  const int n1 = (int)(row % N1);
-  const long long r2 = row / N1;
-  const int n0 = (int)(r2 % N0);
-  const long long bx = r2 / N0;
-  const long long q0 = coil_off ? coil_off[bx] : bx * ns;
-  const long long q1 = coil_off ? coil_off[bx + 1] : q0 + ns;
+  const int cr = c >> LCB, cc = c & (CB - 1);
+  const long long row = (long long)blockIdx.x * RB + cr;
+  const bool live = row < nrows;
+  long long q0 = 0, q1 = 0, goff = 0, pix0 = 0, map0 = 0, opix = 0;
+  float a01 = 0.f;
+  if (live) {
+    const unsigned r2 = (unsigned)row / (unsigned)N1, n1 = (unsigned)row - r2 * N1;  // nrows < 2^31
+    const unsigned bx = r2 / (unsigned)N0, n0 = r2 - bx * N0;
+    q0 = coil_off ? coil_off[bx] : (long long)bx * ns;
+    q1 = coil_off ? coil_off[bx + 1] : q0 + ns;
+    map0 = coil_off ? 0 : bx * ns;
+    goff = ((long long)grid_of(n0, p.G[0], p.c[0]) * p.G[1] + grid_of(n1, p.G[1], p.c[1])) * L;
+    pix0 = ((long long)n0 * N1 + n1) * N2;
+    opix = bx * x_stride + pix0;
+    a01 = p.scale * apod_at(p, 0, n0) * apod_at(p, 1, n1);
+  }
   const long long gsz = (long long)p.G[0] * p.G[1] * L;
-  const long long goff = ((long long)grid_of(n0, p.G[0], p.c[0]) * p.G[1] + grid_of(n1, p.G[1], p.c[1])) * L;
-  const long long pix0 = ((long long)n0 * N1 + n1) * N2;
-  // Short rows (N2 <= 128) use all threads: ng groups of pw threads, group h reduces the
-  // coils c = h, h+ng, ... of each chunk for one pixel per thread; the group sums meet in
-  // LDS at the end. Longer rows: one group, up to kCropMaxPix pixels per thread.
-  const int ng = N2 <= kThreadsFFT / 4 ? 4 : (N2 <= kThreadsFFT / 2 ? 2 : 1);
-  const int pw = kThreadsFFT / ng;
-  const int grp = tid / pw, tin = tid - grp * pw;
-  float2 acc[kCropMaxPix];
-#pragma unroll
-  for (int k = 0; k < kCropMaxPix; ++k) acc[k] = make_float2(0.f, 0.f);
-  for (long long qc = q0; qc < q1; qc += S::NT) {
-    const int nr = (int)min((long long)S::NT, q1 - qc);
-    for (int e = tid; e < S::NT * L; e += kThreadsFFT) {
-      const int c = e / L, j = e - c * L;
-      buf[j * S::NTP + c] = c < nr ? conjf2(grid[(qc + c) * gsz + goff + j]) : make_float2(0.f, 0.f);
+  // chunks of coils: the most any image of the block has, so that every thread reaches
+  // every barrier
+  int nch = (int)((ns + CB - 1) / CB);
+  if (coil_off) {
+    const unsigned per = (unsigned)N0 * N1, last = (unsigned)min(nrows, (long long)(blockIdx.x + 1) * RB) - 1;
+    int most = 0;
+    for (unsigned b = blockIdx.x * RB / per; b <= last / per; ++b) most = max(most, coil_off[b + 1] - coil_off[b]);
+    nch = (most + CB - 1) / CB;
+  }
+  float2* orow = out + opix;
+  auto put = [&](int n2, float2 s) {
+    const float a = a01 * apod_at(p, 2, n2);
+    float2 y = make_float2(s.x * a, s.y * a);
+    if (accumulate) {
+      const float2 o = orow[n2];
+      y.x += o.x;
+      y.y += o.y;
     }
-    __syncthreads();
-    fft_lds<L, S>(buf, tw);
+    orow[n2] = y;
+  };
+  auto term = [&](float2 x, float2 s) {
+    const float2 y = conjf2(x);
+    if (!smaps) return y;
+    return conj_maps ? cmul(y, conjf2(s)) : cmul(y, s);
+  };
+  float2 v[TB::A], x[TB::Z];
+  auto fetch = [&](int k) {
+    const long long qc = q0 + (long long)k * CB + cc;
+    const bool valid = live && qc < q1;
+    const float2* src = grid + (valid ? qc * gsz + goff : 0);  // coils past the last are transformed and not used
+    load_first<L>(v, j, [&](int i, int) { return conjf2(src[i]); });
+  };
+  if (nch > 0) fetch(0);
+  TB::fill(tab, twg, tid, P::T * NT);
+  if constexpr (LCB == 0) {
+    // with no more than one coil the row needs no sum; more (uneven problems) add up in LDS order
+    float2 acc[TB::Z];
 #pragma unroll
-    for (int k = 0; k < kCropMaxPix; ++k) {
-      const int n2 = tin + k * pw;
-      if (n2 < N2) {
-        const int g2 = grid_of(n2, L, p.c[2]);
-        for (int c = grp; c < nr; c += ng) {
-          float2 v = conjf2(buf[g2 * S::NTP + c]);
-          if (smaps) {
-            const float2 s = smaps[(qc + c - (coil_off ? 0 : bx * ns)) * s_stride + pix0 + n2];
-            v = conj_maps ? cmul(v, conjf2(s)) : cmul(v, s);
+    for (int q = 0; q < TB::Z; ++q) acc[q] = make_float2(0.f, 0.f);
+    for (int k = 0; k < nch; ++k) {
+      if (k > 0) {
+        fetch(k);
+        __syncthreads();
+      }
+      finish<L, NT, true, REV>(v, x, buf, tab, j, c);
+      const bool valid = live && q0 + k < q1 && (L / TB::Z == P::T || j < L / TB::Z);
+      auto pix = [&](int q) { return pix_of(j + q * (L / TB::Z), N2, L, p.c[2]); };
+      float2 s[TB::Z];
+      if (smaps) {
+        const float2* srow = smaps + (valid ? (q0 + k - map0) * s_stride + pix0 : 0);
+#pragma unroll
+        for (int q = 0; q < TB::Z; ++q) s[q] = srow[max(pix(q), 0)];
+      }
+#pragma unroll
+      for (int q = 0; q < TB::Z; ++q) {
+        const float2 y = term(x[q], s[q]);
+        const bool in = valid && pix(q) >= 0;
+        acc[q].x = in ? acc[q].x + y.x : acc[q].x;
+        acc[q].y = in ? acc[q].y + y.y : acc[q].y;
+      }
+    }
+    if (live && (L / TB::Z == P::T || j < L / TB::Z)) {
+#pragma unroll
+      for (int q = 0; q < TB::Z; ++q) {
+        const int n2 = pix_of(j + q * (L / TB::Z), N2, L, p.c[2]);
+        if (n2 >= 0) put(n2, acc[q]);
+      }
+    }
+  } else {
+    const int l = cc * P::T + j, pw = GT / ng;
+    const int grp = l / pw, n = l - grp * pw;   // grp == ng for the GT % ng threads left over
+    float2 acc[KM];
+#pragma unroll
+    for (int m = 0; m < KM; ++m) acc[m] = make_float2(0.f, 0.f);
+    for (int k = 0; k < nch; ++k) {
+      if (k > 0) fetch(k);
+      finish<L, NT, true, REV>(v, x, buf, tab, j, c);
+      stage_rows<L, NT, REV>(x, buf, j, c);
+      const long long qk = q0 + (long long)k * CB;
+      const int nr = live && grp < ng ? (int)max(0LL, min((long long)CB, q1 - qk)) : 0;
+#pragma unroll
+      for (int m = 0; m < KM; ++m) {
+        const int n2 = n + m * pw;
+        if (n2 < N2) {
+          const int i = grid_of(n2, L, p.c[2]);
+          const float2* s = smaps + (smaps ? (qk - map0) * s_stride + pix0 + n2 : 0);
+          for (int b = grp; b < nr; b += 4 * ng) {  // four coils' maps in flight
+            float2 sv[4];
+            if (smaps) {
+#pragma unroll
+              for (int u = 0; u < 4; ++u) sv[u] = s[min(b + u * ng, nr - 1) * s_stride];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int bu = b + u * ng;
+              const float2 y = term(buf[LY::at(i, cr * CB + min(bu, nr - 1))], sv[u]);
+              acc[m].x = bu < nr ? acc[m].x + y.x : acc[m].x;
+              acc[m].y = bu < nr ? acc[m].y + y.y : acc[m].y;
+            }
           }
-          acc[k].x += v.x;
-          acc[k].y += v.y;
         }
       }
+      __syncthreads();
     }
-    __syncthreads();
-  }
-  if (ng > 1) {  // one pixel per thread: fold the groups' sums into group 0
-    if (grp > 0 && tin < N2) buf[grp * pw + tin] = acc[0];
-    __syncthreads();
-    if (grp == 0 && tin < N2)
-      for (int h = 1; h < ng; ++h) {
-        const float2 o = buf[h * pw + tin];
-        acc[0].x += o.x;
-        acc[0].y += o.y;
-      }
-  }
-  const float a01 = p.scale * apod_at(p, 0, n0) * apod_at(p, 1, n1);
-  float2* orow = out + bx * x_stride + pix0;
+    if (ng > 1) {  // pw >= N2: one pixel a thread; a row's own part of buf holds its sums
+      float2* part = buf + LY::at(0, cr * CB);
+      if (grp > 0 && grp < ng && n < N2) part[(grp - 1) * N2 + n] = acc[0];
+      __syncthreads();
+      if (grp == 0 && n < N2)
+        for (int h = 1; h < ng; ++h) {
+          const float2 o = part[(h - 1) * N2 + n];
+          acc[0].x += o.x;
+          acc[0].y += o.y;
+        }
+    }
+    if (live && grp == 0) {
 #pragma unroll
-  for (int k = 0; k < kCropMaxPix; ++k) {
-    const int n2 = tin + k * pw;
-    if (grp == 0 && n2 < N2) {
-      const float a = a01 * apod_at(p, 2, n2);
-      float2 v = make_float2(acc[k].x * a, acc[k].y * a);
-      if (accumulate) {
-        const float2 o = orow[n2];
-        v.x += o.x;
-        v.y += o.y;
+      for (int m = 0; m < KM; ++m) {
+        const int n2 = n + m * pw;
+        if (n2 < N2) put(n2, acc[m]);
       }
-      orow[n2] = v;
     }
   }
 }
@@ -278,7 +391,6 @@ int fill_geo(Geo3& p, int ndim, const int* N, const int* G, const int* center, c
       off += n;
     }
   }
-  if (p.N[2] > kCropMaxPix * kThreadsFFT) MRA_FAIL("fused fft: last image dim above 768");
   p.scale = scale;
   return 0;
 }
@@ -296,11 +408,12 @@ int launch_col(int a, float2* grid, const Geo3& p, long long Q, const float2* tw
   const long long outer = a == 0 ? Q : Q * p.N[0];
   const int rc = with_length(p.G[a], [&](auto LL) {
     constexpr int L = decltype(LL)::value;
-    using S = Shape<L, false>;
-    if (inner < S::NT) MRA_FAIL("fused fft: inner extent below the column tile");
-    const long long nb = outer * ((inner + S::NT - 1) / S::NT);
-    if (nb > 0x7fffffffLL) MRA_FAIL("fused fft: grid too large");
-    col_kernel<L, MODE><<<(unsigned)nb, kThreadsFFT, 0, st>>>(grid, p, a, inner, tw, kern);
+    using P = Plan<L>;
+    if (inner < P::NC) MRA_FAIL("fused fft: inner extent below the column tile");
+    if (inner > kMaxInner) MRA_FAIL("fused fft: inner extent too large");
+    const long long nblk = (inner + P::NC - 1) / P::NC;
+    if (outer * nblk > 0x7fffffffLL) MRA_FAIL("fused fft: grid too large");
+    col_kernel<L, MODE><<<(unsigned)(outer * nblk), P::T * P::NC, 0, st>>>(grid, p, a, inner, (unsigned)nblk, tw, kern);
     return 0;
   });
   if (rc < 0) MRA_FAIL("fused fft: length without an LDS plan");
@@ -310,28 +423,50 @@ int launch_col(int a, float2* grid, const Geo3& p, long long Q, const float2* tw
 int launch_pad_rows(const float2* x, long long x_stride, const float2* smaps, long long s_stride, long long ns,
                     const int* img_index, const Geo3& p, long long Q, float2* grid, const float2* tw, hipStream_t st) {
   const long long nrows = Q * p.N[0] * p.N[1];
+  if (nrows > 0x7fffffffLL) MRA_FAIL("fused fft: grid too large");
   const int rc = with_length(p.G[2], [&](auto LL) {
     constexpr int L = decltype(LL)::value;
-    using S = Shape<L, true>;
-    const long long nb = (nrows + S::NT - 1) / S::NT;
-    if (nb > 0x7fffffffLL) MRA_FAIL("fused fft: grid too large");
-    pad_row_kernel<L><<<(unsigned)nb, kThreadsFFT, 0, st>>>(x, x_stride, smaps, s_stride, ns, img_index, p, nrows,
-                                                            grid, tw);
+    using P = Plan<L>;
+    const long long nb = (nrows + P::NR - 1) / P::NR;
+    pad_row_kernel<L><<<(unsigned)nb, P::T * P::NR, 0, st>>>(x, x_stride, smaps, s_stride, ns, img_index, p, nrows,
+                                                             grid, tw);
     return 0;
   });
   if (rc < 0) MRA_FAIL("fused fft: length without an LDS plan");
   return rc;
 }
 
-int launch_crop_rows(const float2* grid, const Geo3& p, long long nx, long long ns, const float2* smaps,
-                     long long s_stride, const int* coil_off, int conj_maps, int accumulate, float2* out,
-                     long long x_stride, const float2* tw, hipStream_t st) {
-  const long long nb = nx * p.N[0] * p.N[1];
-  if (nb > 0x7fffffffLL) MRA_FAIL("fused fft: image too large");
+int launch_crop_rows(const float2* grid, const Geo3& p, long long nq, long long nx, long long ns,
+                     const float2* smaps, long long s_stride, const int* coil_off, int conj_maps, int accumulate,
+                     float2* out, long long x_stride, const float2* tw, hipStream_t st) {
+  const long long nrows = nx * p.N[0] * p.N[1];
+  if (nrows > 0x7fffffffLL) MRA_FAIL("fused fft: image too large");
   const int rc = with_length(p.G[2], [&](auto LL) {
     constexpr int L = decltype(LL)::value;
-    crop_row_kernel<L><<<(unsigned)nb, kThreadsFFT, 0, st>>>(grid, p, ns, smaps, s_stride, coil_off, conj_maps,
-                                                             accumulate, out, x_stride, tw);
+    using P = Plan<L>;
+    // coils of a row at a time: the (mean) coil count rounded up to a power of two, as far
+    // as the block has rows; the rest of the block takes further image rows
+    const long long mean = coil_off ? (nq + nx - 1) / nx : ns;
+    auto run = [&](auto LC) {
+      constexpr int LCB = decltype(LC)::value;
+      if constexpr ((1 << LCB) <= P::NA) {
+        constexpr int CB = 1 << LCB, RB = P::NA / CB;
+        // threads to a pixel: as many as the row has pixels for (one pixel a thread), else one
+        const int ng = max(1, min(CB, P::T * CB / p.N[2]));
+        const long long nb = (nrows + RB - 1) / RB;
+        crop_row_kernel<L, LCB><<<(unsigned)nb, P::T * P::NA, 0, st>>>(grid, p, nrows, ns, smaps, s_stride, coil_off,
+                                                                       ng, conj_maps, accumulate, out, x_stride, tw);
+      }
+    };
+    int lcb = 0;
+    while ((2 << lcb) <= P::NA && lcb < 4 && (1 << lcb) < mean) ++lcb;
+    switch (lcb) {
+      case 0: run(std::integral_constant<int, 0>{}); break;
+      case 1: run(std::integral_constant<int, 1>{}); break;
+      case 2: run(std::integral_constant<int, 2>{}); break;
+      case 3: run(std::integral_constant<int, 3>{}); break;
+      default: run(std::integral_constant<int, 4>{}); break;
+    }
     return 0;
   });
   if (rc < 0) MRA_FAIL("fused fft: length without an LDS plan");
@@ -398,7 +533,7 @@ int mra_fft_crop_adjoint(int ndim, const int* N, const int* G, const int* center
   hipStream_t st = (hipStream_t)stream;
   for (int a = lead; a <= 1; ++a)
     if (launch_col<kAdj>(a, (float2*)grid, p, nq, t[a - lead], nullptr, st)) return 1;
-  if (launch_crop_rows((const float2*)grid, p, nx, ns, (const float2*)smaps, s_stride, coil_off, conj_maps, accumulate,
+  if (launch_crop_rows((const float2*)grid, p, nq, nx, ns, (const float2*)smaps, s_stride, coil_off, conj_maps, accumulate,
                        (float2*)out, x_stride, t[ndim - 1], st))
     return 1;
   MRA_CHECK_LAUNCH("fft_crop_adjoint");
@@ -427,7 +562,7 @@ int mra_toeplitz_fused(int ndim, const int* N, const int* G, const int* center, 
   if (ndim == 3 && launch_col<kFwd>(1, g, p, ns, t[1], nullptr, st)) return 1;
   if (launch_col<kToep>(lead, g, p, ns, t[0], (const float2*)kern, st)) return 1;
   if (ndim == 3 && launch_col<kAdj>(1, g, p, ns, t[1], nullptr, st)) return 1;
-  if (launch_crop_rows(g, p, 1, ns, (const float2*)smaps, s_stride, nullptr, 1, accumulate, (float2*)out, 0,
+  if (launch_crop_rows(g, p, ns, 1, ns, (const float2*)smaps, s_stride, nullptr, 1, accumulate, (float2*)out, 0,
                        t[ndim - 1], st))
     return 1;
   MRA_CHECK_LAUNCH("toeplitz_fused");

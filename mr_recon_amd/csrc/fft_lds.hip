@@ -17,82 +17,71 @@ namespace fft {
 // block. COL: transforms along an axis of stride `inner` (inner >= NT), NT consecutive
 // columns per block.
 template <int L, bool ROW>
-__global__ __launch_bounds__(kThreadsFFT) void fft_axis_kernel(float2* __restrict__ data, long long outer,
-                                                                long long inner, const float2* __restrict__ twg,
-                                                                int inverse) {
-  using S = Shape<L, ROW>;
-  __shared__ float2 buf[L * S::NTP];
-  __shared__ float2 tw[L];
+__global__ __launch_bounds__(Plan<L>::T * (ROW ? Plan<L>::NR : Plan<L>::NC)) void fft_axis_kernel(
+    float2* __restrict__ data, long long outer, long long inner, const float2* __restrict__ twg, int inverse) {
+  using P = Plan<L>;
+  constexpr int NT = ROW ? P::NR : P::NC;
+  constexpr bool REV = ROW && RowOrder<L>::REV;
+  using TB = Tables<L, REV>;
+  __shared__ float2 buf[BufSize<L, NT>::value];
+  __shared__ float2 tab[TB::SIZE];
   const int tid = threadIdx.x;
-  for (int m = tid; m < L; m += kThreadsFFT) tw[m] = twg[m];
-  long long o, i0;
-  int nvalid;
+  const int c = ROW ? tid / P::T : tid % NT, j = ROW ? tid % P::T : tid / NT;
+  bool valid;
+  float2* base;        // rows: this thread's row at j; columns: the block's slab
+  unsigned off = 0, row = 8;
   if constexpr (ROW) {
-    o = (long long)blockIdx.x * S::NT;
-    i0 = 0;
-    nvalid = (int)min((long long)S::NT, outer - o);
+    const long long o = (long long)blockIdx.x * NT + c;
+    valid = o < outer;
+    base = data + (valid ? o * L : 0) + j;
   } else {
-    const long long nblk = (inner + S::NT - 1) / S::NT;
-    o = blockIdx.x / nblk;
-    i0 = (blockIdx.x - o * nblk) * S::NT;
-    nvalid = (int)min((long long)S::NT, inner - i0);
+    const long long nblk = (inner + NT - 1) / NT;
+    const long long o = blockIdx.x / nblk, i0 = (blockIdx.x - o * nblk) * NT;
+    base = data + o * L * inner;
+    valid = i0 + c < inner;
+    row = (unsigned)inner * 8u;
+    off = valid ? j * row + (unsigned)(i0 + c) * 8u : kNone;
   }
+  const Slab slab(data + (ROW ? 0 : base - data), ROW ? 0 : L * row);
   const float sgn = inverse ? -1.0f : 1.0f;  // conj on load and store for the inverse
-  if constexpr (ROW) {
-    const float2* src = data + o * L;
-    for (int e = tid; e < S::NT * L; e += kThreadsFFT) {
-      const int c = e / L, j = e - c * L;
-      if (c < nvalid) {
-        const float2 x = src[(long long)c * L + j];
-        buf[j * S::NTP + c] = make_float2(x.x, sgn * x.y);
+  float2 v[TB::A], x[TB::Z];
+  load_first<L>(v, j, [&](int, int d) { return ROW ? base[d] : slab.load(off, d * row); });
+#pragma unroll
+  for (int q = 0; q < TB::A; ++q) v[q].y *= sgn;
+  TB::fill(tab, twg, tid, P::T * NT);
+  finish<L, NT, ROW, REV>(v, x, buf, tab, j, c);
+  if constexpr (ROW && RowOrder<L>::STAGE) {
+    stage_rows<L, NT, REV>(x, buf, j, c);
+    float2* blk = data + (long long)blockIdx.x * NT * L;
+    for (int e = tid; e < NT * L; e += P::T * NT) {
+      const int r = e / L, i = e - r * L;
+      if ((long long)blockIdx.x * NT + r < outer) {
+        const float2 y = buf[Lay<L, TB::A, NT, true>::at(i, r)];
+        blk[e] = make_float2(y.x, sgn * y.y);
       }
     }
   } else {
-    const float2* src = data + o * L * inner + i0;
-    for (int e = tid; e < S::NT * L; e += kThreadsFFT) {
-      const int j = e / S::NT, c = e - j * S::NT;
-      if (c < nvalid) {
-        const float2 x = src[(long long)j * inner + c];
-        buf[j * S::NTP + c] = make_float2(x.x, sgn * x.y);
-      }
-    }
-  }
-  __syncthreads();
-  fft_lds<L, S>(buf, tw);
-  if constexpr (ROW) {
-    float2* dst = data + o * L;
-    for (int e = tid; e < S::NT * L; e += kThreadsFFT) {
-      const int c = e / L, j = e - c * L;
-      if (c < nvalid) {
-        const float2 x = buf[j * S::NTP + c];
-        dst[(long long)c * L + j] = make_float2(x.x, sgn * x.y);
-      }
-    }
-  } else {
-    float2* dst = data + o * L * inner + i0;
-    for (int e = tid; e < S::NT * L; e += kThreadsFFT) {
-      const int j = e / S::NT, c = e - j * S::NT;
-      if (c < nvalid) {
-        const float2 x = buf[j * S::NTP + c];
-        dst[(long long)j * inner + c] = make_float2(x.x, sgn * x.y);
-      }
-    }
+    emit<L, REV>(x, j, [&](int, int d, float2 y) {
+      y.y *= sgn;
+      if (!ROW) slab.store(off, d * row, y);
+      else if (valid) base[d] = y;
+    });
   }
 }
 
 template <int L>
 int launch_axis(float2* data, long long outer, long long inner, const float2* tw, int inverse, hipStream_t st) {
+  using P = Plan<L>;
   if (inner == 1) {
-    using S = Shape<L, true>;
-    const long long nb = (outer + S::NT - 1) / S::NT;
+    const long long nb = (outer + P::NR - 1) / P::NR;
     if (nb > 0x7fffffffLL) MRA_FAIL("fft: too many transforms");
-    fft_axis_kernel<L, true><<<(unsigned)nb, kThreadsFFT, 0, st>>>(data, outer, inner, tw, inverse);
+    fft_axis_kernel<L, true><<<(unsigned)nb, P::T * P::NR, 0, st>>>(data, outer, inner, tw, inverse);
   } else {
-    using S = Shape<L, false>;
-    if (inner < S::NT) MRA_FAIL("fft: inner extent below the column tile");
-    const long long nb = outer * ((inner + S::NT - 1) / S::NT);
+    if (inner < P::NC) MRA_FAIL("fft: inner extent below the column tile");
+    if (inner > kMaxInner) MRA_FAIL("fft: inner extent too large");
+    const long long nb = outer * ((inner + P::NC - 1) / P::NC);
     if (nb > 0x7fffffffLL) MRA_FAIL("fft: too many transforms");
-    fft_axis_kernel<L, false><<<(unsigned)nb, kThreadsFFT, 0, st>>>(data, outer, inner, tw, inverse);
+    fft_axis_kernel<L, false><<<(unsigned)nb, P::T * P::NC, 0, st>>>(data, outer, inner, tw, inverse);
   }
   MRA_CHECK_LAUNCH("fft axis");
   return 0;
