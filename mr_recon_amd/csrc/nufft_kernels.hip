@@ -232,7 +232,7 @@ __global__ __launch_bounds__(256) void plan_weights_kernel(const float* __restri
   for (int d = 0; d < D; ++d) {
     const float t = tsort[(long long)s * D + d];
     ok = ok && isfinite(t);
-    const int lower = ok ? kb_weights<P>(t, g.r, bt.b[d], 1.0f, w) : 0;
+    const int lower = ok ? kb_weights_fine<P>(t, g.r, bt.b[d], w) : 0;
     const int lw = ok ? pmod(lower + g.wrap[d], g.G[d]) % T : 0;
     base = base * SUB + lw;
 #pragma unroll
