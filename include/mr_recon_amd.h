@@ -178,6 +178,23 @@ int mra_toeplitz_fused(int ndim, const int* N, const int* G, const int* center, 
                        long long ns, long long s_stride, const void* kern, void* work, int accumulate, void* out,
                        const void* const* tw, void* stream);
 
+/* The same transforms for any lengths 2..640 (mra_fft_any_supported): tw[d] = device copy of
+ * mra_fft_any_table(G[d]), mra_fft_any_table_len(G[d]) complex values. One image batch, no
+ * per-problem indexing; mra_fft_crop_adjoint_any takes nx * ns grids. */
+int mra_fft_any_supported(int ndim, const int* G);
+long long mra_fft_any_table_len(int L);
+int mra_fft_any_table(int L, float* host);
+int mra_fft_pad_forward_any(int ndim, const int* N, const int* G, const int* center, const void* x, long long x_stride,
+                            const void* smaps, long long ns, long long s_stride, long long nq, const float* apod,
+                            float scale, void* grid, const void* const* tw, void* stream);
+int mra_fft_crop_adjoint_any(int ndim, const int* N, const int* G, const int* center, void* grid, long long nx,
+                             const void* smaps, long long ns, long long s_stride, int conj_maps, const float* apod,
+                             float scale, int accumulate, void* out, long long x_stride, const void* const* tw,
+                             void* stream);
+int mra_toeplitz_any(int ndim, const int* N, const int* G, const int* center, const void* x, const void* smaps,
+                     long long ns, long long s_stride, const void* kern, void* work, int accumulate, void* out,
+                     const void* const* tw, void* stream);
+
 /* ---- nearest-grid sampling ------------------------------------------------------------------
  * Gather / scatter-add at one flat grid index per sample: gridded_nufft's forward_interp_only
  * and adjoint_grid_only (fourier.py:1250-1294, via indexing.multi_index / multi_grid,

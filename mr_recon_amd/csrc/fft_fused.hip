@@ -23,6 +23,7 @@
 // NUFFT.normal_toeplitz (fourier.py:302-352) with SENSE expand / reduce
 // (linops.py:1161, 1220, 1265-1306).
 #include "capi_util.h"
+#include "fft_any.h"
 #include "fft_lds.h"
 
 namespace mra {
@@ -369,6 +370,250 @@ __global__ __launch_bounds__(Plan<L>::T * Plan<L>::NA) void crop_row_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same three kernels for run-time lengths (fft_any.h); dynamic LDS: M * (NT + 1) points of
+// the transforms, then the M roots. Copies between memory and LDS issue four loads at a time.
+
+template <int TPB, int NT, bool BLUE>
+__global__ __launch_bounds__(TPB) void any_pad_row_kernel(const float2* __restrict__ x, long long x_stride,
+                                                          const float2* __restrict__ smaps, long long s_stride,
+                                                          long long ns, Geo3 p, AnyPlan ap, long long nrows,
+                                                          float2* __restrict__ grid, const float2* __restrict__ tab) {
+  using A = Any<TPB, NT>;
+  extern __shared__ float2 buf[];
+  float2* tw = buf + ap.M * A::NTP;
+  __shared__ long long rsrc[NT], rmap[NT], rdst[NT];
+  __shared__ float rapo[NT];
+  const int tid = threadIdx.x, L = ap.L;
+  const long long row0 = (long long)blockIdx.x * NT;
+  const int N0 = p.N[0], N1 = p.N[1], N2 = p.N[2];
+  if (tid < NT) {
+    const unsigned row = (unsigned)min(row0 + tid, nrows - 1);  // nrows < 2^31; rows past the last are not stored
+    const unsigned r2 = row / (unsigned)N1, n1 = row - r2 * N1;
+    const unsigned q = r2 / (unsigned)N0, n0 = r2 - q * N0;
+    const unsigned bq = q / (unsigned)ns;
+    const long long pix = ((long long)n0 * N1 + n1) * N2;
+    rsrc[tid] = bq * x_stride + pix;
+    rmap[tid] = (q - bq * (unsigned)ns) * s_stride + pix;
+    rapo[tid] = p.scale * apod_at(p, 0, n0) * apod_at(p, 1, n1);
+    rdst[tid] = (((long long)q * p.G[0] + grid_of(n0, p.G[0], p.c[0])) * p.G[1] + grid_of(n1, p.G[1], p.c[1])) * L;
+  }
+  for (int m = tid; m < ap.M; m += TPB) tw[m] = tab[m];
+  __syncthreads();
+  const int n = NT * L;
+  for (int e0 = tid; e0 < n; e0 += 4 * TPB) {
+    float2 v[4], s[4];
+    float a[4];
+    int c[4], i[4], n2[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = min(e0 + u * TPB, n - 1);
+      c[u] = (int)__umulhi((unsigned)e, ap.inv_l);
+      i[u] = e - c[u] * L;
+      n2[u] = pix_of(i[u], N2, L, p.c[2]);
+      v[u] = x[rsrc[c[u]] + max(n2[u], 0)];
+    }
+    if (smaps) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s[u] = smaps[rmap[c[u]] + max(n2[u], 0)];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) a[u] = rapo[c[u]] * apod_at(p, 2, max(n2[u], 0));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float2 y = smaps ? cmul(v[u], s[u]) : v[u];
+      if (e0 + u * TPB < n)
+        buf[i[u] * A::NTP + c[u]] = n2[u] >= 0 ? make_float2(y.x * a[u], y.y * a[u]) : make_float2(0.f, 0.f);
+    }
+  }
+  __syncthreads();
+  A::template transform<BLUE>(buf, tw, tab, ap);
+  for (int e = tid; e < n; e += TPB) {
+    const int c = (int)__umulhi((unsigned)e, ap.inv_l), i = e - c * L;
+    if (row0 + c < nrows) grid[rdst[c] + i] = buf[i * A::NTP + c];
+  }
+}
+
+template <int TPB, int NT, bool BLUE, int MODE>
+__global__ __launch_bounds__(TPB) void any_col_kernel(float2* __restrict__ grid, Geo3 p, AnyPlan ap, int axis,
+                                                      long long inner, unsigned nblk, const float2* __restrict__ tab,
+                                                      const float2* __restrict__ kern) {
+  using A = Any<TPB, NT>;
+  extern __shared__ float2 buf[];
+  float2* tw = buf + ap.M * A::NTP;
+  const int tid = threadIdx.x, L = ap.L;
+  const unsigned o = blockIdx.x / nblk;
+  const long long col0 = (long long)(blockIdx.x - o * nblk) * NT;
+  long long base;
+  if (axis == 0) {
+    base = (long long)o * L * inner;
+  } else {  // axis 1: o = q * N0 + n0
+    const unsigned q = o / (unsigned)p.N[0];
+    const int n0 = (int)(o - q * p.N[0]);
+    base = ((long long)q * p.G[0] + grid_of(n0, p.G[0], p.c[0])) * (long long)L * inner;
+  }
+  const int Na = p.N[axis], ca = p.c[axis];
+  const unsigned row = (unsigned)inner * 8u;
+  const Slab g(grid + base, L * row);
+  // a thread's column is the same at every step (TPB % NT == 0)
+  const int c = tid % NT;
+  const unsigned off = col0 + c < inner ? (unsigned)(col0 + c) * 8u : kNone;
+  const int j0 = tid / NT;
+  constexpr int JS = TPB / NT;
+  for (int j = j0; j < L; j += 4 * JS) {
+    float2 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = j + u * JS;
+      const bool in = i < L && (MODE == kAdj || pix_of(i, Na, L, ca) >= 0) && off != kNone;
+      v[u] = g.load(in ? off + i * row : kNone, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (j + u * JS < L) buf[(j + u * JS) * A::NTP + c] = MODE == kAdj ? conjf2(v[u]) : v[u];
+  }
+  for (int m = tid; m < ap.M; m += TPB) tw[m] = tab[m];
+  __syncthreads();
+  A::template transform<BLUE>(buf, tw, tab, ap);
+  if constexpr (MODE == kToep) {
+    const Slab ks(kern, L * row);
+    for (int j = j0; j < L; j += 4 * JS) {
+      float2 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int i = j + u * JS;
+        v[u] = ks.load(i < L && off != kNone ? off + i * row : kNone, 0);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (j + u * JS < L) {
+          float2& y = buf[(j + u * JS) * A::NTP + c];
+          y = conjf2(cmul(y, v[u]));
+        }
+    }
+    __syncthreads();
+    A::template transform<BLUE>(buf, tw, tab, ap);
+  }
+  for (int j = j0; j < L; j += JS) {
+    const float2 y = buf[j * A::NTP + c];
+    const bool in = (MODE == kFwd || pix_of(j, Na, L, ca) >= 0) && off != kNone;
+    g.store(in ? off + j * row : kNone, 0, MODE == kFwd ? y : conjf2(y));
+  }
+}
+
+// NT / 2^lcb image rows per block, 2^lcb coils of each at a time; more than one chunk of
+// coils only where 2^lcb == NT (one row), whose pixels' sums stay in registers.
+template <int TPB, int NT, bool BLUE>
+__global__ __launch_bounds__(TPB) void any_crop_row_kernel(const float2* __restrict__ grid, Geo3 p, AnyPlan ap,
+                                                           long long nrows, int ns, const float2* __restrict__ smaps,
+                                                           long long s_stride, int lcb, int conj_maps, int accumulate,
+                                                           float2* __restrict__ out, long long x_stride,
+                                                           const float2* __restrict__ tab) {
+  using A = Any<TPB, NT>;
+  extern __shared__ float2 buf[];
+  float2* tw = buf + ap.M * A::NTP;
+  __shared__ long long rgrid[NT], rpix[NT], rout[NT];
+  __shared__ float rapo[NT];
+  constexpr int KM = (kAnyMax + TPB - 1) / TPB;
+  const int tid = threadIdx.x, L = ap.L;
+  const int N0 = p.N[0], N1 = p.N[1], N2 = p.N[2];
+  const int cb = 1 << lcb, rb = NT >> lcb;
+  const long long row0 = (long long)blockIdx.x * rb;
+  const long long gsz = (long long)p.G[0] * p.G[1] * L;
+  if (tid < rb) {
+    const unsigned row = (unsigned)min(row0 + tid, nrows - 1);
+    const unsigned r2 = row / (unsigned)N1, n1 = row - r2 * N1;
+    const unsigned bx = r2 / (unsigned)N0, n0 = r2 - bx * N0;
+    const long long pix = ((long long)n0 * N1 + n1) * N2;
+    rgrid[tid] = (long long)bx * ns * gsz + ((long long)grid_of(n0, p.G[0], p.c[0]) * p.G[1] + grid_of(n1, p.G[1], p.c[1])) * L;
+    rpix[tid] = pix;
+    rout[tid] = bx * x_stride + pix;
+    rapo[tid] = p.scale * apod_at(p, 0, n0) * apod_at(p, 1, n1);
+  }
+  for (int m = tid; m < ap.M; m += TPB) tw[m] = tab[m];
+  __syncthreads();
+  const int n = NT * L;
+  auto put = [&](int r, int n2, float2 s) {
+    if (row0 + r >= nrows) return;
+    const float a = rapo[r] * apod_at(p, 2, n2);
+    float2 y = make_float2(s.x * a, s.y * a);
+    float2* o = out + rout[r] + n2;
+    if (accumulate) {
+      y.x += o->x;
+      y.y += o->y;
+    }
+    *o = y;
+  };
+  // sum over the chunk's coils [q0, q0 + nr) of pixel n2 of row r
+  auto coils = [&](int r, int n2, int q0, int nr) {
+    const int at = grid_of(n2, L, p.c[2]) * A::NTP + r * cb;
+    const float2* s = smaps ? smaps + q0 * s_stride + rpix[r] + n2 : nullptr;
+    float2 acc = make_float2(0.f, 0.f);
+    for (int b = 0; b < nr; b += 4) {
+      float2 sv[4];
+      if (smaps) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sv[u] = s[min(b + u, nr - 1) * s_stride];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        float2 y = conjf2(buf[at + min(b + u, nr - 1)]);
+        if (smaps) y = conj_maps ? cmul(y, conjf2(sv[u])) : cmul(y, sv[u]);
+        acc.x = b + u < nr ? acc.x + y.x : acc.x;
+        acc.y = b + u < nr ? acc.y + y.y : acc.y;
+      }
+    }
+    return acc;
+  };
+  float2 acc[KM];
+#pragma unroll
+  for (int m = 0; m < KM; ++m) acc[m] = make_float2(0.f, 0.f);
+  for (int q0 = 0; q0 < ns; q0 += cb) {
+    const int nr = min(cb, ns - q0);
+    for (int e0 = tid; e0 < n; e0 += 4 * TPB) {
+      float2 v[4];
+      int at[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int e = min(e0 + u * TPB, n - 1);
+        const int c = (int)__umulhi((unsigned)e, ap.inv_l), i = e - c * L;
+        at[u] = i * A::NTP + c;
+        v[u] = grid[rgrid[c >> lcb] + (q0 + min(c & (cb - 1), nr - 1)) * gsz + i];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (e0 + u * TPB < n) buf[at[u]] = conjf2(v[u]);
+    }
+    __syncthreads();
+    A::template transform<BLUE>(buf, tw, tab, ap);
+    if (cb < NT) {
+      const int np = rb * N2;
+      for (int e = tid; e < np; e += TPB) {
+        const int r = e / N2, n2 = e - r * N2;
+        put(r, n2, coils(r, n2, q0, nr));
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < KM; ++m) {
+        const int n2 = tid + m * TPB;
+        if (n2 < N2) {
+          const float2 y = coils(0, n2, q0, nr);
+          acc[m].x += y.x;
+          acc[m].y += y.y;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (cb == NT) {
+#pragma unroll
+    for (int m = 0; m < KM; ++m) {
+      const int n2 = tid + m * TPB;
+      if (n2 < N2) put(0, n2, acc[m]);
+    }
+  }
+}
+
 int fill_geo(Geo3& p, int ndim, const int* N, const int* G, const int* center, const float* apod, float scale) {
   if (ndim < 1 || ndim > 3) MRA_FAIL("fused fft: ndim must be 1..3");
   const int lead = 3 - ndim;
@@ -402,10 +647,46 @@ long long inner_of(const Geo3& p, int a) {
   return in;
 }
 
+// Whether axis a runs on its compiled plan: the length has one and the axis is the last or
+// has columns for the tile.
+bool compiled(const Geo3& p, int a) { return plan_supported(p.G[a]) && (a == 2 || inner_of(p, a) >= 64); }
+
+// Kernels with more than 64 KB of LDS have to say so once.
+template <class K>
+int allow_lds(K kernel, size_t bytes) {
+  if (bytes <= 64 * 1024) return 0;
+  if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    MRA_FAIL("fused fft: LDS size refused");
+  }
+  return 0;
+}
+
+template <int MODE>
+int launch_col_any(int a, float2* grid, const Geo3& p, long long Q, const float2* tab, const float2* kern,
+                   hipStream_t st) {
+  const AnyPlan* ap = any_plan(p.G[a]);
+  if (!ap) MRA_FAIL("fused fft: length outside 2..640");
+  const long long inner = inner_of(p, a);
+  if (inner > kMaxInner) MRA_FAIL("fused fft: inner extent too large");
+  const long long outer = a == 0 ? Q : Q * p.N[0];
+  return with_any(*ap, [&](auto TPB, auto NT, auto BL) {
+    constexpr int tpb = decltype(TPB)::value, nt = decltype(NT)::value;
+    const size_t lds = any_shape(*ap).lds;
+    const long long nblk = (inner + nt - 1) / nt;
+    if (outer * nblk > 0x7fffffffLL) MRA_FAIL("fused fft: grid too large");
+    auto k = any_col_kernel<tpb, nt, decltype(BL)::value, MODE>;
+    if (allow_lds(k, lds)) return 1;
+    k<<<(unsigned)(outer * nblk), tpb, lds, st>>>(grid, p, *ap, a, inner, (unsigned)nblk, tab, kern);
+    return 0;
+  });
+}
+
 template <int MODE>
 int launch_col(int a, float2* grid, const Geo3& p, long long Q, const float2* tw, const float2* kern, hipStream_t st) {
   const long long inner = inner_of(p, a);
   const long long outer = a == 0 ? Q : Q * p.N[0];
+  if (!compiled(p, a)) return launch_col_any<MODE>(a, grid, p, Q, tw, kern, st);
   const int rc = with_length(p.G[a], [&](auto LL) {
     constexpr int L = decltype(LL)::value;
     using P = Plan<L>;
@@ -424,6 +705,18 @@ int launch_pad_rows(const float2* x, long long x_stride, const float2* smaps, lo
                     const int* img_index, const Geo3& p, long long Q, float2* grid, const float2* tw, hipStream_t st) {
   const long long nrows = Q * p.N[0] * p.N[1];
   if (nrows > 0x7fffffffLL) MRA_FAIL("fused fft: grid too large");
+  if (!compiled(p, 2)) {
+    const AnyPlan* ap = any_plan(p.G[2]);
+    if (!ap || img_index) MRA_FAIL("fused fft: length without an LDS plan");
+    return with_any(*ap, [&](auto TPB, auto NT, auto BL) {
+      constexpr int tpb = decltype(TPB)::value, nt = decltype(NT)::value;
+      const size_t lds = any_shape(*ap).lds;
+      auto k = any_pad_row_kernel<tpb, nt, decltype(BL)::value>;
+      if (allow_lds(k, lds)) return 1;
+      k<<<(unsigned)((nrows + nt - 1) / nt), tpb, lds, st>>>(x, x_stride, smaps, s_stride, ns, p, *ap, nrows, grid, tw);
+      return 0;
+    });
+  }
   const int rc = with_length(p.G[2], [&](auto LL) {
     constexpr int L = decltype(LL)::value;
     using P = Plan<L>;
@@ -441,6 +734,23 @@ int launch_crop_rows(const float2* grid, const Geo3& p, long long nq, long long 
                      float2* out, long long x_stride, const float2* tw, hipStream_t st) {
   const long long nrows = nx * p.N[0] * p.N[1];
   if (nrows > 0x7fffffffLL) MRA_FAIL("fused fft: image too large");
+  if (!compiled(p, 2)) {
+    const AnyPlan* ap = any_plan(p.G[2]);
+    if (!ap || coil_off) MRA_FAIL("fused fft: length without an LDS plan");
+    if (ns > 0x7fffffffLL) MRA_FAIL("fused fft: too many maps");
+    return with_any(*ap, [&](auto TPB, auto NT, auto BL) {
+      constexpr int tpb = decltype(TPB)::value, nt = decltype(NT)::value;
+      int lcb = 0;
+      while ((2 << lcb) <= nt && (1 << lcb) < ns) ++lcb;
+      const size_t lds = any_shape(*ap).lds;
+      const long long rb = nt >> lcb, nb = (nrows + rb - 1) / rb;
+      auto k = any_crop_row_kernel<tpb, nt, decltype(BL)::value>;
+      if (allow_lds(k, lds)) return 1;
+      k<<<(unsigned)nb, tpb, lds, st>>>(grid, p, *ap, nrows, (int)ns, smaps, s_stride, lcb, conj_maps, accumulate, out,
+                                        x_stride, tw);
+      return 0;
+    });
+  }
   const int rc = with_length(p.G[2], [&](auto LL) {
     constexpr int L = decltype(LL)::value;
     using P = Plan<L>;
@@ -494,13 +804,43 @@ int mra_fft_fused_supported(int ndim, const int* G) {
   return 1;
 }
 
+// 1 when the *_any entry points support grids of shape G: every length in 2..640.
+int mra_fft_any_supported(int ndim, const int* G) {
+  if (ndim < 1 || ndim > 3) return 0;
+  for (int d = 0; d < ndim; ++d)
+    if (!fft::any_plan(G[d])) return 0;
+  return 1;
+}
+
+// Device table of length L for the *_any entry points: complex values, and their contents
+// (host memory). For lengths with a compiled plan the first L values are mra_fft_lds_twiddles'.
+long long mra_fft_any_table_len(int L) {
+  const fft::AnyPlan* p = fft::any_plan(L);
+  return p ? fft::any_table_len(*p) : 0;
+}
+
+int mra_fft_any_table(int L, float* host) {
+  MRA_TRY_BEGIN
+  const fft::AnyPlan* p = fft::any_plan(L);
+  if (!p) MRA_FAIL("fft: length outside 2..640");
+  try {
+    fft::any_table(*p, host);
+  } catch (...) {
+    MRA_FAIL("fft: out of memory for a table");
+  }
+  MRA_TRY_END
+}
+
+}  // extern "C"
+
+namespace {
+
 // Forward: grid[q] = FFT(pad(x[img(q)] * S[map(q)] * apod * scale)), q < nq, with
 // img(q) = img_index[q] or q / ns, map(q) = q or q % ns. tw[d] as for mra_fft_lds.
-int mra_fft_pad_forward(int ndim, const int* N, const int* G, const int* center, const void* x, long long x_stride,
+int pad_forward(int ndim, const int* N, const int* G, const int* center, const void* x, long long x_stride,
                         const void* smaps, long long ns, long long s_stride, const int* img_index, long long nq,
                         const float* apod, float scale, void* grid, const void* const* tw, void* stream) {
   MRA_TRY_BEGIN
-  if (!mra_fft_fused_supported(ndim, G)) MRA_FAIL("fused fft: grid shape not supported");
   if (nq < 1 || ns < 1) MRA_FAIL("fused fft: batch sizes must be positive");
   Geo3 p{};
   if (fill_geo(p, ndim, N, G, center, apod, scale)) return 1;
@@ -519,12 +859,11 @@ int mra_fft_pad_forward(int ndim, const int* N, const int* G, const int* center,
 // Adjoint: out[bx] (+)= scale * apod * sum_{q of bx} crop(iFFT(grid[q])) * (conj) S[q],
 // grids of image bx = coil_off[bx] .. coil_off[bx+1]-1 or bx*ns .. bx*ns+ns-1; nq grids
 // in all. The grids are overwritten.
-int mra_fft_crop_adjoint(int ndim, const int* N, const int* G, const int* center, void* grid, long long nq,
+int crop_adjoint(int ndim, const int* N, const int* G, const int* center, void* grid, long long nq,
                          long long nx, const void* smaps, long long ns, long long s_stride, const int* coil_off,
                          int conj_maps, const float* apod, float scale, int accumulate, void* out,
                          long long x_stride, const void* const* tw, void* stream) {
   MRA_TRY_BEGIN
-  if (!mra_fft_fused_supported(ndim, G)) MRA_FAIL("fused fft: grid shape not supported");
   if (nq < 1 || nx < 1 || ns < 1) MRA_FAIL("fused fft: batch sizes must be positive");
   Geo3 p{};
   if (fill_geo(p, ndim, N, G, center, apod, scale)) return 1;
@@ -543,12 +882,10 @@ int mra_fft_crop_adjoint(int ndim, const int* N, const int* G, const int* center
 // Toeplitz normal operator of one image x and ns maps (2D / 3D):
 // out (+)= sum_q conj(S[q]) crop(iFFT(K * FFT(pad(x * S[q])))), K the PSF spectrum in
 // the unshifted layout on grid G (normalisation folded in). work holds ns grids.
-int mra_toeplitz_fused(int ndim, const int* N, const int* G, const int* center, const void* x, const void* smaps,
+int toeplitz(int ndim, const int* N, const int* G, const int* center, const void* x, const void* smaps,
                        long long ns, long long s_stride, const void* kern, void* work, int accumulate, void* out,
                        const void* const* tw, void* stream) {
   MRA_TRY_BEGIN
-  if (ndim < 2) MRA_FAIL("fused Toeplitz: 2D or 3D only");
-  if (!mra_fft_fused_supported(ndim, G)) MRA_FAIL("fused fft: grid shape not supported");
   if (ns < 1) MRA_FAIL("fused fft: batch sizes must be positive");
   Geo3 p{};
   if (fill_geo(p, ndim, N, G, center, nullptr, 1.0f)) return 1;
@@ -567,6 +904,61 @@ int mra_toeplitz_fused(int ndim, const int* N, const int* G, const int* center, 
     return 1;
   MRA_CHECK_LAUNCH("toeplitz_fused");
   MRA_TRY_END
+}
+
+}  // namespace
+
+extern "C" {
+
+// The compiled grids only (mra_fft_fused_supported), tw[d] as for mra_fft_lds.
+int mra_fft_pad_forward(int ndim, const int* N, const int* G, const int* center, const void* x, long long x_stride,
+                        const void* smaps, long long ns, long long s_stride, const int* img_index, long long nq,
+                        const float* apod, float scale, void* grid, const void* const* tw, void* stream) {
+  if (!mra_fft_fused_supported(ndim, G)) MRA_FAIL("fused fft: grid shape not supported");
+  return pad_forward(ndim, N, G, center, x, x_stride, smaps, ns, s_stride, img_index, nq, apod, scale, grid, tw, stream);
+}
+
+int mra_fft_crop_adjoint(int ndim, const int* N, const int* G, const int* center, void* grid, long long nq,
+                         long long nx, const void* smaps, long long ns, long long s_stride, const int* coil_off,
+                         int conj_maps, const float* apod, float scale, int accumulate, void* out,
+                         long long x_stride, const void* const* tw, void* stream) {
+  if (!mra_fft_fused_supported(ndim, G)) MRA_FAIL("fused fft: grid shape not supported");
+  return crop_adjoint(ndim, N, G, center, grid, nq, nx, smaps, ns, s_stride, coil_off, conj_maps, apod, scale,
+                      accumulate, out, x_stride, tw, stream);
+}
+
+int mra_toeplitz_fused(int ndim, const int* N, const int* G, const int* center, const void* x, const void* smaps,
+                       long long ns, long long s_stride, const void* kern, void* work, int accumulate, void* out,
+                       const void* const* tw, void* stream) {
+  if (ndim < 2) MRA_FAIL("fused Toeplitz: 2D or 3D only");
+  if (!mra_fft_fused_supported(ndim, G)) MRA_FAIL("fused fft: grid shape not supported");
+  return toeplitz(ndim, N, G, center, x, smaps, ns, s_stride, kern, work, accumulate, out, tw, stream);
+}
+
+// Any grid with lengths 2..640 (mra_fft_any_supported), tw[d] = device copy of
+// mra_fft_any_table(G[d]). One image batch with the same maps (no per-problem indexing).
+int mra_fft_pad_forward_any(int ndim, const int* N, const int* G, const int* center, const void* x, long long x_stride,
+                            const void* smaps, long long ns, long long s_stride, long long nq, const float* apod,
+                            float scale, void* grid, const void* const* tw, void* stream) {
+  if (!mra_fft_any_supported(ndim, G)) MRA_FAIL("fused fft: grid shape not supported");
+  return pad_forward(ndim, N, G, center, x, x_stride, smaps, ns, s_stride, nullptr, nq, apod, scale, grid, tw, stream);
+}
+
+int mra_fft_crop_adjoint_any(int ndim, const int* N, const int* G, const int* center, void* grid, long long nx,
+                             const void* smaps, long long ns, long long s_stride, int conj_maps, const float* apod,
+                             float scale, int accumulate, void* out, long long x_stride, const void* const* tw,
+                             void* stream) {
+  if (!mra_fft_any_supported(ndim, G)) MRA_FAIL("fused fft: grid shape not supported");
+  return crop_adjoint(ndim, N, G, center, grid, nx * ns, nx, smaps, ns, s_stride, nullptr, conj_maps, apod, scale,
+                      accumulate, out, x_stride, tw, stream);
+}
+
+int mra_toeplitz_any(int ndim, const int* N, const int* G, const int* center, const void* x, const void* smaps,
+                     long long ns, long long s_stride, const void* kern, void* work, int accumulate, void* out,
+                     const void* const* tw, void* stream) {
+  if (ndim < 2) MRA_FAIL("fused Toeplitz: 2D or 3D only");
+  if (!mra_fft_any_supported(ndim, G)) MRA_FAIL("fused fft: grid shape not supported");
+  return toeplitz(ndim, N, G, center, x, smaps, ns, s_stride, kern, work, accumulate, out, tw, stream);
 }
 
 }  // extern "C"

@@ -191,9 +191,39 @@ __device__ __forceinline__ void dft(float2 (&v)[R]) {
     v[4] = make_float2(m1.x - n1.y, m1.y + n1.x);
     v[2] = make_float2(m2.x + n2.y, m2.y - n2.x);
     v[3] = make_float2(m2.x - n2.y, m2.y + n2.x);
+  } else if constexpr (R == 7 || R == 11 || R == 13) {
+    // odd prime: sums and differences of the pairs (p, R - p); real cosines and sines
+    constexpr auto w = roots<R>();
+    constexpr int H = (R - 1) / 2;
+    float2 t[H], d[H];
+    float2 s = v[0];
+#pragma unroll
+    for (int p = 0; p < H; ++p) {
+      t[p] = make_float2(v[p + 1].x + v[R - 1 - p].x, v[p + 1].y + v[R - 1 - p].y);
+      d[p] = make_float2(v[p + 1].x - v[R - 1 - p].x, v[p + 1].y - v[R - 1 - p].y);
+      s.x += t[p].x;
+      s.y += t[p].y;
+    }
+    const float2 a0 = v[0];
+    v[0] = s;
+#pragma unroll
+    for (int q = 1; q <= H; ++q) {
+      float2 a = a0, b = make_float2(0.f, 0.f);
+#pragma unroll
+      for (int p = 0; p < H; ++p) {
+        const float c = w.re[(p + 1) * q % R], z = w.im[(p + 1) * q % R];  // z = -sin
+        a.x += c * t[p].x;
+        a.y += c * t[p].y;
+        b.x += z * d[p].x;
+        b.y += z * d[p].y;
+      }
+      // a + i b, a - i b
+      v[q] = make_float2(a.x - b.y, a.y + b.x);
+      v[R - q] = make_float2(a.x + b.y, a.y - b.x);
+    }
   } else {
     // composite: R = A B, n = B n1 + n2, k = k1 + A k2
-    constexpr int A = R == 10 || R == 15 || R == 20 ? 5 : 4, B = R / A;
+    constexpr int A = R == 10 || R == 15 || R == 20 ? 5 : R == 9 ? 3 : 4, B = R / A;
     static_assert(A * B == R, "radix");
     float2 u[B][A];
     unroll<B>([&](auto N2) {

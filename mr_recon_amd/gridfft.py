@@ -73,6 +73,34 @@ class _LdsFFT:
 _lds_fft = _LdsFFT()
 
 
+class _AnyFFT:
+    """Device tables of the fused transforms of run-time length, per (device, length)."""
+
+    def __init__(self):
+        self._tab: dict = {}
+        self._arr: dict = {}
+        self._lock = threading.Lock()
+
+    def tables(self, device: torch.device, shape: tuple):
+        key = (device.index, shape)
+        with self._lock:
+            arr = self._arr.get(key)
+            if arr is None:
+                tabs = []
+                for L in shape:
+                    t = self._tab.get((device.index, L))
+                    if t is None:
+                        host = torch.empty(2 * int(lib().mra_fft_any_table_len(L)), dtype=torch.float32)
+                        check(lib().mra_fft_any_table(L, ctypes.cast(host.data_ptr(), ctypes.POINTER(ctypes.c_float))))
+                        t = self._tab[(device.index, L)] = host.to(device)
+                    tabs.append(t)
+                arr = self._arr[key] = (tabs, (ctypes.c_void_p * len(shape))(*[t.data_ptr() for t in tabs]))
+            return arr[1]
+
+
+_any_fft = _AnyFFT()
+
+
 def _fft_inplace(x: torch.Tensor, d: int, inverse: bool) -> torch.Tensor:
     _lib.require_device(x)
     if x.dtype != torch.complex64 or not x.is_contiguous():

@@ -239,6 +239,7 @@ def crop_reduce(grid: torch.Tensor, im_size, grid_size, nx: int, smaps: torch.Te
 
 
 _fused_ok: dict = {}
+_any_ok: dict = {}
 
 
 def fused_supported(grid_size) -> bool:
@@ -251,6 +252,17 @@ def fused_supported(grid_size) -> bool:
     return ok
 
 
+def fused_any_supported(grid_size) -> bool:
+    """Whether the fused transforms cover grids of this shape on run-time plans (any lengths
+    2..640), for one image batch; grids with compiled plans (``fused_supported``) use those."""
+    key = tuple(int(g) for g in grid_size)
+    ok = _any_ok.get(key)
+    if ok is None:
+        ok = bool(lib().mra_fft_any_supported(len(key), _lib.ints(key)))
+        _any_ok[key] = ok
+    return ok
+
+
 def pad_fft(x: torch.Tensor, im_size, grid_size, smaps: torch.Tensor | None = None,
             apod: torch.Tensor | None = None, scale: float = 1.0, center=None,
             img_index: torch.Tensor | None = None, nq: int | None = None,
@@ -259,11 +271,12 @@ def pad_fft(x: torch.Tensor, im_size, grid_size, smaps: torch.Tensor | None = No
     grid tensor (nx[, C], *G), unnormalised, unshifted layout: new, or written into
     ``out`` (contiguous complex64 with as many elements). With ``img_index`` (batched
     problems), grid q pads image img_index[q] times map q (nq grids)."""
-    from .gridfft import _fftn, _lds_fft
+    from .gridfft import _any_fft, _fftn, _lds_fft
 
     D = len(im_size)
     G = tuple(int(g) for g in grid_size)
-    if not fused_supported(G):
+    compiled = fused_supported(G)
+    if not compiled and (img_index is not None or not fused_any_supported(G)):
         if img_index is not None:
             raise ValueError("pad_fft: batched padding needs a grid with an LDS FFT plan")
         g = pad_expand(x, im_size, G, smaps=smaps, apod=apod, scale=scale, center=center)
@@ -306,6 +319,11 @@ def pad_fft(x: torch.Tensor, im_size, grid_size, smaps: torch.Tensor | None = No
             raise ValueError("pad_fft: bad output tensor")
         out = out.view(shape)
     cen = None if center is None else _lib.ints(center)
+    if not compiled:
+        check(lib().mra_fft_pad_forward_any(D, _lib.ints(im_size), _lib.ints(G), cen, ptr(x), npix, ptr(smaps), ns, npix,
+                                            q, ptr(apod), float(scale), ptr(out), _any_fft.tables(x.device, G),
+                                            stream_ptr(x.device)))
+        return out
     check(lib().mra_fft_pad_forward(D, _lib.ints(im_size), _lib.ints(G), cen, ptr(x), npix, ptr(smaps), ns, npix,
                                     ptr(img_index), q, ptr(apod), float(scale), ptr(out),
                                     _lds_fft.tables(x.device, G), stream_ptr(x.device)))
@@ -319,11 +337,12 @@ def ifft_crop(grid: torch.Tensor, im_size, grid_size, nx: int, smaps: torch.Tens
     """crop_reduce(iFFT(grid)) (unnormalised inverse) into image (nx, *N). The grid is
     used as work space and overwritten. With ``coil_off`` (batched problems), image i
     reduces grids and maps coil_off[i] .. coil_off[i+1]-1."""
-    from .gridfft import _ifftn, _lds_fft
+    from .gridfft import _any_fft, _ifftn, _lds_fft
 
     D = len(im_size)
     G = tuple(int(g) for g in grid_size)
-    if not fused_supported(G):
+    compiled = fused_supported(G)
+    if not compiled and (coil_off is not None or not grid.is_contiguous() or not fused_any_supported(G)):
         if coil_off is not None:
             raise ValueError("ifft_crop: batched reduction needs a grid with an LDS FFT plan")
         g = _ifftn(grid.reshape(-1, *G), D)
@@ -354,6 +373,11 @@ def ifft_crop(grid: torch.Tensor, im_size, grid_size, nx: int, smaps: torch.Tens
     elif out.numel() != nx * npix or out.dtype != torch.complex64 or not out.is_contiguous():
         raise ValueError("ifft_crop: bad output tensor")
     cen = None if center is None else _lib.ints(center)
+    if not compiled:
+        check(lib().mra_fft_crop_adjoint_any(D, _lib.ints(im_size), _lib.ints(G), cen, ptr(grid), nx, ptr(smaps), ns,
+                                             npix, int(conj_maps), ptr(apod), float(scale), int(accumulate), ptr(out),
+                                             npix, _any_fft.tables(grid.device, G), stream_ptr(grid.device)))
+        return out
     check(lib().mra_fft_crop_adjoint(D, _lib.ints(im_size), _lib.ints(G), cen, ptr(grid), nq, nx, ptr(smaps), ns,
                                      npix, ptr(coil_off), int(conj_maps), ptr(apod), float(scale), int(accumulate),
                                      ptr(out), npix, _lds_fft.tables(grid.device, G), stream_ptr(grid.device)))
@@ -364,14 +388,15 @@ def toeplitz_normal(x: torch.Tensor, im_size, grid_size, smaps: torch.Tensor, ke
                     center=None, out: torch.Tensor | None = None, accumulate: bool = False) -> torch.Tensor:
     """sum_c conj(S_c) crop(iFFT(K * FFT(pad(x S_c)))) for one image x (*N) and maps (C, *N),
     K the PSF multiplier on grid ``grid_size`` (unshifted layout, normalisation included)."""
-    from .gridfft import _fftn, _ifftn, _lds_fft
+    from .gridfft import _any_fft, _fftn, _ifftn, _lds_fft
 
     D = len(im_size)
     G = tuple(int(g) for g in grid_size)
     x = _c64(x, "x").reshape(1, *im_size)
     smaps = _c64(smaps, "smaps")
     C = int(math.prod(smaps.shape[:-D]))
-    if D < 2 or not fused_supported(G):
+    compiled = D >= 2 and fused_supported(G)
+    if not compiled and (D < 2 or tuple(kern_unshifted.shape) != G or not fused_any_supported(G)):
         g = pad_expand(x, im_size, G, smaps=smaps, center=center)
         g = _fftn(g.reshape(C, *G), D)
         cmul_bcast(g, kern_unshifted)
@@ -390,9 +415,9 @@ def toeplitz_normal(x: torch.Tensor, im_size, grid_size, smaps: torch.Tensor, ke
         raise ValueError("toeplitz_normal: bad output tensor")
     work = torch.empty((C, *G), dtype=torch.complex64, device=x.device)
     cen = None if center is None else _lib.ints(center)
-    check(lib().mra_toeplitz_fused(D, _lib.ints(im_size), _lib.ints(G), cen, ptr(x), ptr(smaps), C, npix, ptr(kern),
-                                   ptr(work), int(accumulate), ptr(out), _lds_fft.tables(x.device, G),
-                                   stream_ptr(x.device)))
+    run, tab = (lib().mra_toeplitz_fused, _lds_fft) if compiled else (lib().mra_toeplitz_any, _any_fft)
+    check(run(D, _lib.ints(im_size), _lib.ints(G), cen, ptr(x), ptr(smaps), C, npix, ptr(kern), ptr(work),
+              int(accumulate), ptr(out), tab.tables(x.device, G), stream_ptr(x.device)))
     return out
 
 
