@@ -35,7 +35,7 @@ from . import _lib, ops
 from ._lib import check, lib, ptr, stream_ptr
 from .dtypes import complex_dtype
 from .fourier import _fftn, _ifftn, hip_nufft
-from .plan import make_geoms
+from .plan import batch_samples_per_item, make_geoms
 
 
 @dataclass
@@ -115,6 +115,8 @@ class BatchedSense:
         if tile == "auto":
             tile, self.tile_times = self._tune_tile(problems, oversamp, width, samples_per_item)
         self.problems = list(problems)
+        if samples_per_item is None:
+            samples_per_item = batch_samples_per_item(sum(pr.trj.numel() // 2 for pr in self.problems))
         sizes = {}
         for i, pr in enumerate(self.problems):
             _lib.require_device(pr.trj, pr.mps)

@@ -817,10 +817,8 @@ constexpr int kReduceBatch = MRA_REDUCE_BATCH;
 #define MRA_REDUCE_AHEAD 4
 #endif
 constexpr int kReduceAhead = MRA_REDUCE_AHEAD;  // items whose loads are issued together (2D)
-#ifndef MRA_REDUCE_AHEAD3
-#define MRA_REDUCE_AHEAD3 2
-#endif
-constexpr int kReduceAhead3 = MRA_REDUCE_AHEAD3;  // further items of one tile issued together (3D)
+// Items loaded together by a 3D thread of RB batch entries.
+constexpr int reduce_ahead3(int rb) { return rb == 1 ? 8 : 2; }
 
 // grid_reduce for 2D with every G >= SUB and even G[1]: the T x T tile has T*T/2 point
 // pairs (y, x), (y, x + 1), x even; thread t owns pair t % (T*T/2) for batch entries
@@ -952,16 +950,22 @@ __device__ __forceinline__ void reduce_pairs_2d(float2* __restrict__ grid, const
   }
 }
 
-// grid_reduce for 3D with every G >= SUB and even G[2]: thread t owns the points
-// (z, y, x), (z, y, x + 1) of the output tile, x even, for kReduceBatch batch entries;
-// each covering item's pair is one 16-byte load per entry.
-template <int P, int T>
+// Two neighbouring points along the last dim, at any 8-byte alignment.
+struct __attribute__((aligned(8))) Pair { float x, y, z, w; };
+
+// grid_reduce for 3D with every G >= SUB: thread t owns the points (z, y, x), (z, y, x + 1) of
+// the output tile, x even, for RB batch entries; each covering item's pair is one 16-byte load
+// per entry. A launch lasts as long as its hottest tile (the k-space centre of a kooshball of
+// 4001 spokes is covered by 333 items), so a tile's further items go AH at a time.
+// Odd G[2] takes the same path (90x104x77 x 7 coils, width 6, grid edge 97: 553 -> 206 us): past
+// the wrap a pair may start at the subgrid's last point (loaded one back and shifted) and the
+// grid's last pair has one point.
+template <int P, int T, int RB, int AH, bool SHIFT>
 __device__ __forceinline__ void reduce_pairs_3d(float2* __restrict__ grid, const float2* __restrict__ sbase,
                                                 const Geom& g, const int (&tc)[3], const int (&cand)[3][3],
                                                 const int (&ncand)[3], const int* __restrict__ titems, int b0,
                                                 int nb, int accumulate) {
   using TS = TileShape<3, P, T>;
-  constexpr int RB = kReduceBatch;
   const int t = threadIdx.x;
   const int xp = t % (T / 2), rest = t / (T / 2);
   const int gc[3] = {tc[0] * T + rest / T, tc[1] * T + rest % T, tc[2] * T + 2 * xp};
@@ -969,89 +973,91 @@ __device__ __forceinline__ void reduce_pairs_3d(float2* __restrict__ grid, const
   float4 acc[RB];
 #pragma unroll
   for (int b = 0; b < RB; ++b) acc[b] = make_float4(0.f, 0.f, 0.f, 0.f);
-  auto add = [&](const float4 (&v)[RB]) {
+  auto add = [&](const Pair (&v)[RB], bool past) {
+    const bool shift = SHIFT && past;
 #pragma unroll
     for (int b = 0; b < RB; ++b) {
-      acc[b].x += v[b].x;
-      acc[b].y += v[b].y;
-      acc[b].z += v[b].z;
-      acc[b].w += v[b].w;
+      acc[b].x += shift ? v[b].z : v[b].x;
+      acc[b].y += shift ? v[b].w : v[b].y;
+      acc[b].z += shift ? 0.f : v[b].z;
+      acc[b].w += shift ? 0.f : v[b].w;
     }
   };
-  auto load = [&](int it, int e, float4 (&v)[RB]) {
+  auto load = [&](int it, int e, Pair (&v)[RB]) {
     const float2* slot = sbase + ((long long)(it - g.item_base) * g.nbatch + b0) * TS::SUBN + e;
 #pragma unroll
-    for (int b = 0; b < RB; ++b)
-      v[b] = b < nb ? *(const float4*)(slot + (long long)b * TS::SUBN) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int b = 0; b < RB; ++b) v[b] = b < nb ? *(const Pair*)(slot + (long long)b * TS::SUBN) : Pair{0.f, 0.f, 0.f, 0.f};
   };
   // Covering tiles in row-major order, each tile's items in order (the sums' order). The
-  // first items of two neighbouring tiles along dim 2 are loaded together, further items
-  // (split hot tiles) two at a time, so that a block does not wait out one load per item.
+  // first items of two neighbouring tiles along dim 2 are loaded together.
   for (int k0 = 0; k0 < ncand[0]; ++k0)
     for (int k1 = 0; k1 < ncand[1]; ++k1)
       for (int k2 = 0; k2 < ncand[2]; k2 += 2) {
         int e[2], i0[2], i1[2];
+        bool sh[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           const bool valid = k2 + j < ncand[2];
           const int c0 = cand[0][k0], c1 = cand[1][k1], c2 = cand[2][valid ? k2 + j : k2];
           const int l0 = pmod(gc[0] - c0 * T, g.G[0]), l1 = pmod(gc[1] - c1 * T, g.G[1]);
-          const int l2 = pmod(gc[2] - c2 * T, g.G[2]);  // even, so l2 + 1 < SUB when l2 < SUB
+          const int l2 = pmod(gc[2] - c2 * T, g.G[2]);
           const bool ok = valid && inside && l0 < TS::SUB && l1 < TS::SUB && l2 < TS::SUB;
-          e[j] = (l0 * TS::SUB + l1) * TS::SUB + l2;
+          sh[j] = SHIFT && l2 == TS::SUB - 1;
+          e[j] = (l0 * TS::SUB + l1) * TS::SUB + l2 - sh[j];
           const int stile = (c0 * g.ntile[1] + c1) * g.ntile[2] + c2;
           i0[j] = ok ? titems[stile] : 0;
           i1[j] = ok ? titems[stile + 1] : 0;
         }
-        float4 first[2][RB];
+        Pair first[2][RB];
 #pragma unroll
         for (int j = 0; j < 2; ++j)
           if (i0[j] < i1[j]) load(i0[j], e[j], first[j]);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           if (i0[j] >= i1[j]) continue;
-          add(first[j]);
+          add(first[j], sh[j]);
           int it = i0[j] + 1;
-          if constexpr (kReduceAhead3 >= 2)
-            for (; it + 2 <= i1[j]; it += 2) {
-              float4 v0[RB], v1[RB];
-              load(it, e[j], v0);
-              load(it + 1, e[j], v1);
-              add(v0);
-              add(v1);
-            }
+          for (; it + AH <= i1[j]; it += AH) {
+            Pair v[AH][RB];
+#pragma unroll
+            for (int u = 0; u < AH; ++u) load(it + u, e[j], v[u]);
+#pragma unroll
+            for (int u = 0; u < AH; ++u) add(v[u], sh[j]);
+          }
           for (; it < i1[j]; ++it) {
-            float4 v0[RB];
-            load(it, e[j], v0);
-            add(v0);
+            Pair v[RB];
+            load(it, e[j], v);
+            add(v, sh[j]);
           }
         }
       }
   if (!inside) return;
+  const bool second = gc[2] + 1 < g.G[2];
   const long long lin = ((long long)gc[0] * g.G[1] + gc[1]) * g.G[2] + gc[2];
 #pragma unroll
   for (int b = 0; b < RB; ++b) {
     if (b >= nb) break;
-    float4* o = (float4*)(grid + g.grid_off + (long long)(b0 + b) * g.grid_stride + lin);
+    float2* o = grid + g.grid_off + (long long)(b0 + b) * g.grid_stride + lin;
     if (accumulate) {
-      const float4 v = *o;
-      acc[b].x += v.x;
-      acc[b].y += v.y;
-      acc[b].z += v.z;
-      acc[b].w += v.w;
+      acc[b].x += o[0].x;
+      acc[b].y += o[0].y;
+      if (second) {
+        acc[b].z += o[1].x;
+        acc[b].w += o[1].y;
+      }
     }
-    *o = acc[b];
+    if (second) *(Pair*)o = Pair{acc[b].x, acc[b].y, acc[b].z, acc[b].w};
+    else *o = make_float2(acc[b].x, acc[b].y);
   }
 }
 
-template <int D, int P, int T>
+template <int D, int P, int T, int RB>
 __global__ __launch_bounds__(kThreads) void grid_reduce_kernel(float2* __restrict__ grid,
                                                                const float2* __restrict__ scratch,
                                                                const Geom* __restrict__ geoms, int prob0,
                                                                int ntiles, const int* __restrict__ tile_items,
                                                                int accumulate) {
   using TS = TileShape<D, P, T>;
-  constexpr int RB = kReduceBatch;
   constexpr int NQ = (TS::TN + kThreads - 1) / kThreads;
   const int prob = prob0 + blockIdx.x / ntiles;
   const int tile = blockIdx.x - (prob - prob0) * ntiles;
@@ -1108,13 +1114,12 @@ __global__ __launch_bounds__(kThreads) void grid_reduce_kernel(float2* __restric
       return;
     }
   }
-  if constexpr (D == 3 && T % 2 == 0 && TS::SUB % 2 == 0 && TS::TN == 2 * kThreads) {
-    // two adjacent points along the last dim per thread, 16-byte loads and stores; needs
-    // even offsets so that a pair never straddles the wrap and stays 16-byte aligned
-    const bool pairs = simple && g.G[2] % 2 == 0 && g.scratch_off % 2 == 0 && g.grid_off % 2 == 0 &&
-                       g.grid_stride % 2 == 0 && (uintptr_t)grid % 16 == 0 && (uintptr_t)scratch % 16 == 0;
-    if (pairs) {
-      reduce_pairs_3d<P, T>(grid, sbase, g, tc, cand, ncand, titems, b0, nb, accumulate);
+  if constexpr (D == 3 && TS::TN == 2 * kThreads) {
+    if (simple) {
+      if (TS::SUB % 2 == 0 && g.G[2] % 2 == 0)
+        reduce_pairs_3d<P, T, RB, reduce_ahead3(RB), false>(grid, sbase, g, tc, cand, ncand, titems, b0, nb, accumulate);
+      else
+        reduce_pairs_3d<P, T, RB, reduce_ahead3(RB), true>(grid, sbase, g, tc, cand, ncand, titems, b0, nb, accumulate);
       return;
     }
   }
@@ -1486,8 +1491,12 @@ static int launch_op(const LaunchArgs& a) {
         return 1;
       }
       dim3 grd((unsigned)((long long)a.ntiles * a.nprob), (unsigned)ngroups);
-      grid_reduce_kernel<D, P, T><<<grd, kThreads, 0, a.stream>>>((float2*)a.dst, (const float2*)a.src, a.geoms,
-                                                                  a.prob, a.ntiles, a.tile_items, a.accumulate);
+      // one entry (a density weight, a single coil): nothing to share a thread with, so that more
+      // items are loaded together instead (96^3 grid, 1.5 M samples: 53 -> 33 us)
+      auto kernel = D == 3 && a.nbatch == 1 ? grid_reduce_kernel<D, P, T, D == 3 ? 1 : kReduceBatch>
+                                            : grid_reduce_kernel<D, P, T, kReduceBatch>;
+      kernel<<<grd, kThreads, 0, a.stream>>>((float2*)a.dst, (const float2*)a.src, a.geoms, a.prob, a.ntiles,
+                                             a.tile_items, a.accumulate);
       break;
     }
     case Op::Grad: {

@@ -42,11 +42,20 @@ def binning_chunk(npts: int, ntiles: int, tile: int, ndim: int) -> int:
     return min(c, 4096)
 
 
-def default_samples_per_item(npts: int) -> int:
-    """Work-item size: about a thousand items per trajectory, 256..8192 samples each."""
+def default_samples_per_item(npts: int, ndim: int = 2) -> int:
+    """Work-item size: about a thousand items per trajectory, 256..8192 samples each; in 3D at
+    most 2560, so that the tiles of the k-space centre do not end a launch alone (5.12 M samples,
+    32 coils: gridding 3.62 -> 3.47 ms against 5120 samples an item)."""
     s = -(-npts // 1024)
     s = -(-s // 256) * 256
-    return int(min(max(s, 256), 8192))
+    return int(min(max(s, 256), 2560 if ndim == 3 else 8192))
+
+
+def batch_samples_per_item(npts: int) -> int:
+    """Work-item size of problems that share their launches, ``npts`` samples in all: other
+    problems' items fill the device, so an item may be longer, which saves partial subgrids
+    (24 problems of 20..130 k samples: 14.5 ms at 256 samples, 12.8 at 512, 12.5 at 1024)."""
+    return min(default_samples_per_item(npts // 2), 1024)
 
 
 def kernel_points(width: float) -> int:
@@ -117,7 +126,7 @@ class SamplePlan:
             pass
         self.ntile = [(g + self.tile - 1) // self.tile for g in self.grid_size]
         self.ntiles = int(math.prod(self.ntile))
-        self.S = int(samples_per_item or default_samples_per_item(self.npts))
+        self.S = int(samples_per_item or default_samples_per_item(self.npts, D))
         if self.S < 1:
             raise ValueError("samples_per_item must be positive")
         self.wrap = tuple(int(w) for w in (wrap if wrap is not None else (0,) * D))
