@@ -5,7 +5,7 @@
 // 7 coils, width 6; 0.50 ms here. 230x187, 11 coils: 86 and 49 us).
 //
 // NT transforms of a block sit in LDS as [point][transform]. Lengths whose prime factors are
-// at most 13 take Stockham passes of radix 2..16 (fewest passes, then smallest radices), in
+// at most 19 take Stockham passes of radix 2..19 (fewest passes, then smallest radices), in
 // place: a pass reads its inputs into registers, synchronises and writes. Other lengths go
 // through Bluestein's chirp-z form (L. Bluestein, "A linear filtering approach to the
 // computation of discrete Fourier transform", IEEE Trans. Audio Electroacoust. 18, 1970) as a
@@ -77,17 +77,17 @@ inline bool best_radices(int n, const int* set, int nset, std::vector<int>& cur,
 }
 
 inline bool make_any_plan(int L, AnyPlan& p) {
-  static const int all[] = {16, 15, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+  static const int all[] = {19, 17, 16, 15, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2};
   p = AnyPlan{};
   if (L < 2 || L > kAnyMax) return false;
   p.L = p.M = L;
   std::vector<int> cur, best;
-  if (!best_radices(L, all, 14, cur, best)) {
+  if (!best_radices(L, all, 16, cur, best)) {
     // convolution length: least (M times passes) among the smooth ones from 2 L - 1 up
     double cost = 1e30;
     for (int M = 2 * L - 1; M <= 2 * kAnyMax && M < 3 * L; ++M) {
       std::vector<int> c2, b2;
-      if (!best_radices(M, all, 14, c2, b2) || !any_shape(M, b2.data(), (int)b2.size()).tpb) continue;
+      if (!best_radices(M, all + 2, 14, c2, b2) || !any_shape(M, b2.data(), (int)b2.size()).tpb) continue;
       const double k = (double)M * (b2.size() + 1);
       if (k < cost) {
         cost = k;
@@ -162,6 +162,10 @@ inline const AnyPlan* any_plan(int L) {
   return L >= 2 && L <= kAnyMax && plans[L].L ? &plans[L] : nullptr;
 }
 
+// What a kernel is compiled for: direct passes up to radix 16, the chirp-z form over them, and
+// direct passes with radix 17 or 19 (whose registers halve the blocks of a CU at 1024 threads).
+enum AnyKind { kDirect = 0, kChirp = 1, kPrime = 2 };
+
 template <int TPB, int NT>
 struct Any {
   static constexpr int NTP = NT + 1;
@@ -199,6 +203,7 @@ struct Any {
   }
 
   // Forward transform of length M of the NT columns, tw = its M roots in LDS.
+  template <bool PRIME>
   static __device__ __forceinline__ void smooth(float2* buf, const float2* tw, const AnyPlan& p) {
     for (int i = 0; i < p.npass; ++i) {
       const int ns = p.ns[i];
@@ -214,17 +219,19 @@ struct Any {
         MRA_ANY_RADIX(8) MRA_ANY_RADIX(9) MRA_ANY_RADIX(10) MRA_ANY_RADIX(11) MRA_ANY_RADIX(12) MRA_ANY_RADIX(13)
         MRA_ANY_RADIX(15) MRA_ANY_RADIX(16)
 #undef MRA_ANY_RADIX
+        case 17: if constexpr (PRIME) pass<17>(buf, tw, tid, M, ns, inv); break;
+        case 19: if constexpr (PRIME) pass<19>(buf, tw, tid, M, ns, inv); break;
       }
     }
   }
 
   // Forward transform of length L of the NT columns of buf (points 0 .. L - 1), in place.
   // tab: the length's device table. The caller has synchronised after writing buf and tw.
-  template <bool BLUE>
+  template <int KIND>
   static __device__ __forceinline__ void transform(float2* buf, const float2* tw, const float2* __restrict__ tab,
                                                    const AnyPlan& p) {
-    if constexpr (!BLUE) {
-      smooth(buf, tw, p);
+    if constexpr (KIND != kChirp) {
+      smooth<KIND == kPrime>(buf, tw, p);
     } else {
       const float2 *chirp = tab + p.M, *conv = chirp + p.L;
       for (int e = threadIdx.x; e < NT * p.M; e += TPB) {
@@ -232,14 +239,14 @@ struct Any {
         buf[at] = j < p.L ? cmul(buf[at], chirp[j]) : make_float2(0.f, 0.f);
       }
       __syncthreads();
-      smooth(buf, tw, p);
+      smooth<false>(buf, tw, p);
       for (int e = threadIdx.x; e < NT * p.M; e += TPB) {
         const int j = e / NT, at = j * NTP + e % NT;
         const float2 y = cmul(buf[at], conv[j]);
         buf[at] = make_float2(y.x, -y.y);
       }
       __syncthreads();
-      smooth(buf, tw, p);
+      smooth<false>(buf, tw, p);
       for (int e = threadIdx.x; e < NT * p.L; e += TPB) {
         const int j = e / NT, at = j * NTP + e % NT;
         const float2 y = buf[at];
@@ -250,13 +257,17 @@ struct Any {
   }
 };
 
-// f(integral_constant<TPB>, integral_constant<NT>, bool_constant<BLUE>) for a plan's shape.
+// f(integral_constant<TPB>, integral_constant<NT>, integral_constant<KIND>) for a plan's shape.
 template <class F>
 int with_any(const AnyPlan& p, F&& f) {
-  const AnyShape s = any_shape(p);
-  const bool blue = p.M != p.L;
-  auto go = [&](auto TPB, auto NT) { return blue ? f(TPB, NT, std::true_type{}) : f(TPB, NT, std::false_type{}); };
   using std::integral_constant;
+  const AnyShape s = any_shape(p);
+  bool prime = false;
+  for (int i = 0; i < p.npass; ++i) prime = prime || p.radix[i] > 16;
+  auto go = [&](auto TPB, auto NT) {
+    if (p.M != p.L) return f(TPB, NT, integral_constant<int, kChirp>{});
+    return prime ? f(TPB, NT, integral_constant<int, kPrime>{}) : f(TPB, NT, integral_constant<int, kDirect>{});
+  };
   if (s.nt == 8) return go(integral_constant<int, 1024>{}, integral_constant<int, 8>{});
   if (s.tpb == 256) return go(integral_constant<int, 256>{}, integral_constant<int, 16>{});
   if (s.tpb == 512) return go(integral_constant<int, 512>{}, integral_constant<int, 16>{});

@@ -374,7 +374,7 @@ __global__ __launch_bounds__(Plan<L>::T * Plan<L>::NA) void crop_row_kernel(
 // The same three kernels for run-time lengths (fft_any.h); dynamic LDS: M * (NT + 1) points of
 // the transforms, then the M roots. Copies between memory and LDS issue four loads at a time.
 
-template <int TPB, int NT, bool BLUE>
+template <int TPB, int NT, int KIND>
 __global__ __launch_bounds__(TPB) void any_pad_row_kernel(const float2* __restrict__ x, long long x_stride,
                                                           const float2* __restrict__ smaps, long long s_stride,
                                                           long long ns, Geo3 p, AnyPlan ap, long long nrows,
@@ -427,14 +427,14 @@ __global__ __launch_bounds__(TPB) void any_pad_row_kernel(const float2* __restri
     }
   }
   __syncthreads();
-  A::template transform<BLUE>(buf, tw, tab, ap);
+  A::template transform<KIND>(buf, tw, tab, ap);
   for (int e = tid; e < n; e += TPB) {
     const int c = (int)__umulhi((unsigned)e, ap.inv_l), i = e - c * L;
     if (row0 + c < nrows) grid[rdst[c] + i] = buf[i * A::NTP + c];
   }
 }
 
-template <int TPB, int NT, bool BLUE, int MODE>
+template <int TPB, int NT, int KIND, int MODE>
 __global__ __launch_bounds__(TPB) void any_col_kernel(float2* __restrict__ grid, Geo3 p, AnyPlan ap, int axis,
                                                       long long inner, unsigned nblk, const float2* __restrict__ tab,
                                                       const float2* __restrict__ kern) {
@@ -474,7 +474,7 @@ __global__ __launch_bounds__(TPB) void any_col_kernel(float2* __restrict__ grid,
   }
   for (int m = tid; m < ap.M; m += TPB) tw[m] = tab[m];
   __syncthreads();
-  A::template transform<BLUE>(buf, tw, tab, ap);
+  A::template transform<KIND>(buf, tw, tab, ap);
   if constexpr (MODE == kToep) {
     const Slab ks(kern, L * row);
     for (int j = j0; j < L; j += 4 * JS) {
@@ -492,7 +492,7 @@ __global__ __launch_bounds__(TPB) void any_col_kernel(float2* __restrict__ grid,
         }
     }
     __syncthreads();
-    A::template transform<BLUE>(buf, tw, tab, ap);
+    A::template transform<KIND>(buf, tw, tab, ap);
   }
   for (int j = j0; j < L; j += JS) {
     const float2 y = buf[j * A::NTP + c];
@@ -503,7 +503,7 @@ __global__ __launch_bounds__(TPB) void any_col_kernel(float2* __restrict__ grid,
 
 // NT / 2^lcb image rows per block, 2^lcb coils of each at a time; more than one chunk of
 // coils only where 2^lcb == NT (one row), whose pixels' sums stay in registers.
-template <int TPB, int NT, bool BLUE>
+template <int TPB, int NT, int KIND>
 __global__ __launch_bounds__(TPB) void any_crop_row_kernel(const float2* __restrict__ grid, Geo3 p, AnyPlan ap,
                                                            long long nrows, int ns, const float2* __restrict__ smaps,
                                                            long long s_stride, int lcb, int conj_maps, int accumulate,
@@ -585,7 +585,7 @@ __global__ __launch_bounds__(TPB) void any_crop_row_kernel(const float2* __restr
         if (e0 + u * TPB < n) buf[at[u]] = conjf2(v[u]);
     }
     __syncthreads();
-    A::template transform<BLUE>(buf, tw, tab, ap);
+    A::template transform<KIND>(buf, tw, tab, ap);
     if (cb < NT) {
       const int np = rb * N2;
       for (int e = tid; e < np; e += TPB) {

@@ -24,7 +24,7 @@ CASES = [
     ((20, 31), (26, 49), 5), ((230, 187), (288, 234), 3), ((64, 50), (64, 63), 1), ((33, 47), (320, 59), 2),
     ((90, 100), (121, 169), 17), ((400, 20), (630, 22), 2), ((2, 3), (3, 5), 1), ((50, 512), (61, 637), 4),
     ((9, 10, 11), (12, 13, 14), 33), ((30, 26, 24), (37, 33, 31), 7), ((20, 16, 24), (25, 64, 40), 2),
-    ((7, 5, 64), (11, 10, 160), 9), ((64, 5, 7), (128, 7, 11), 1),
+    ((7, 5, 64), (11, 10, 160), 9), ((60, 40), (136, 95), 3), ((11, 70), (17, 323), 2), ((64, 5, 7), (128, 7, 11), 1),
 ]
 
 
