@@ -68,6 +68,9 @@ int mra_plan_weights(int ndim, int P, const float* tsort, int npts, const int* G
  * with a per-dimension `param`, as type3_nufft grids on (linops.py:250-251, 311-312). */
 int mra_plan_weights_dims(int ndim, int P, const float* tsort, int npts, const int* G, const int* wrap, float width,
                           const float* betas, float* wsort, int* lbase, void* stream);
+/* The same with the shapes in 64 bits (plans use this one). */
+int mra_plan_weights_dims64(int ndim, int P, const float* tsort, int npts, const int* G, const int* wrap, float width,
+                            const double* betas, float* wsort, int* lbase, void* stream);
 
 /* ---- interpolation / gridding -----------------------------------------------------------
  * mra_interp replaces ungrid (ungrid.py:34-124, Triton kernels _ungrid1d/2d/3d

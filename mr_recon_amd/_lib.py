@@ -45,6 +45,7 @@ SIGNATURES = {
     "mra_geom_fill": (_i, [_vp, _ll, _ll, _ll, _ll, _ll, _i, _i, _i, _ip, _i, _ip, _f, _f, _f, _i, _ll, _i]),
     "mra_plan_weights": (_i, [_i, _i, _vp, _i, _ip, _ip, _f, _f, _vp, _vp, _vp]),
     "mra_plan_weights_dims": (_i, [_i, _i, _vp, _i, _ip, _ip, _f, _fp, _vp, _vp, _vp]),
+    "mra_plan_weights_dims64": (_i, [_i, _i, _vp, _i, _ip, _ip, _f, C.POINTER(C.c_double), _vp, _vp, _vp]),
     "mra_scan_workspace": (_ll, [_ll]),
     "mra_scan_excl_i32": (_i, [_vp, _ll, _vp, _vp, _vp]),
     "mra_bin_workspace": (_ll, [_i, _ll, _ll, _i, _i]),
@@ -180,6 +181,11 @@ class tile_scope:
 def ints(vals) -> C.Array:
     vals = [int(v) for v in vals]
     return (C.c_int * len(vals))(*vals)
+
+
+def doubles(vals) -> C.Array:
+    vals = [float(v) for v in vals]
+    return (C.c_double * len(vals))(*vals)
 
 
 def floats(vals) -> C.Array:

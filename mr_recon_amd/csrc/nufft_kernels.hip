@@ -212,12 +212,13 @@ __device__ __forceinline__ float4 patch_sum_pair(const float4* sb, const float (
 }
 
 // --------------------------------------------------------------------------------------------
-// Kaiser-Bessel shape per dimension (all equal except for sigpy-style per-dim kernels).
+// Kaiser-Bessel shape per dimension (all equal except for sigpy-style per-dim kernels), as
+// (beta / r)^2 in two floats: a beta rounded to 32 bits scales every weight alike (2e-7 a
+// dimension at width 4, oversampling 1.25).
 struct DimBetas {
-  float b[kMaxDim];
+  float kh[kMaxDim], kl[kMaxDim];
 };
 
-// Per sorted sample: KB weights along each dim (unscaled) and the subgrid base offset.
 template <int D, int P, int T>
 __global__ __launch_bounds__(256) void plan_weights_kernel(const float* __restrict__ tsort, int npts, Geom g,
                                                            DimBetas bt, float* __restrict__ wsort,
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(256) void plan_weights_kernel(const float* __restri
   for (int d = 0; d < D; ++d) {
     const float t = tsort[(long long)s * D + d];
     ok = ok && isfinite(t);
-    const int lower = ok ? kb_weights_fine<P>(t, g.r, bt.b[d], w) : 0;
+    const int lower = ok ? kb_weights_fine<P>(t, g.r, bt.kh[d], bt.kl[d], w) : 0;
     const int lw = ok ? pmod(lower + g.wrap[d], g.G[d]) % T : 0;
     base = base * SUB + lw;
 #pragma unroll
@@ -1758,13 +1759,17 @@ int mra_geom_set_ksp_plan_order(void* geom_host, int on) {
 }
 
 // Per sorted sample KB weights (npts x ndim x P floats) and subgrid offsets.
-int mra_plan_weights_dims(int ndim, int P, const float* tsort, int npts, const int* G, const int* wrap, float width,
-                          const float* betas, float* wsort, int* lbase, void* stream) {
+int mra_plan_weights_dims64(int ndim, int P, const float* tsort, int npts, const int* G, const int* wrap, float width,
+                            const double* betas, float* wsort, int* lbase, void* stream) {
   MRA_TRY_BEGIN
   if (ndim < 1 || ndim > 3) MRA_FAIL("plan_weights: ndim must be 1..3");
   if (!betas) MRA_FAIL("plan_weights: null betas");
   LaunchArgs a{};
-  for (int d = 0; d < kMaxDim; ++d) a.betas.b[d] = betas[d < ndim ? d : 0];
+  for (int d = 0; d < kMaxDim; ++d) {
+    const double k = betas[d < ndim ? d : 0] / (0.5f * width);
+    a.betas.kh[d] = (float)(k * k);
+    a.betas.kl[d] = (float)(k * k - a.betas.kh[d]);
+  }
   a.op = Op::Weights;
   a.src = tsort;
   a.dst = wsort;
@@ -1775,9 +1780,20 @@ int mra_plan_weights_dims(int ndim, int P, const float* tsort, int npts, const i
     a.geom.wrap[d] = (d < ndim && wrap) ? wrap[d] : 0;
   }
   a.geom.r = 0.5f * width;
-  a.geom.beta = betas[0];
+  a.geom.beta = (float)betas[0];
   a.stream = (hipStream_t)stream;
   return dispatch(ndim, P, a);
+  MRA_TRY_END
+}
+
+int mra_plan_weights_dims(int ndim, int P, const float* tsort, int npts, const int* G, const int* wrap, float width,
+                          const float* betas, float* wsort, int* lbase, void* stream) {
+  MRA_TRY_BEGIN
+  if (ndim < 1 || ndim > 3) MRA_FAIL("plan_weights: ndim must be 1..3");
+  if (!betas) MRA_FAIL("plan_weights: null betas");
+  double b[kMaxDim];
+  for (int d = 0; d < kMaxDim; ++d) b[d] = betas[d < ndim ? d : 0];
+  return mra_plan_weights_dims64(ndim, P, tsort, npts, G, wrap, width, b, wsort, lbase, stream);
   MRA_TRY_END
 }
 

@@ -162,9 +162,9 @@ class SamplePlan:
         self.wsort = torch.empty(self.npts * D * self.P, dtype=torch.float32, device=dev)
         self.lbase = torch.empty(self.npts, dtype=torch.int32, device=dev)
         with _lib.tile_scope(D, self.tile):
-            check(L.mra_plan_weights_dims(D, self.P, ptr(self.tsort), self.npts, _lib.ints(self.grid_size),
-                                          _lib.ints(self.wrap), self.width, _lib.floats(self.betas),
-                                          ptr(self.wsort), ptr(self.lbase), st))
+            check(L.mra_plan_weights_dims64(D, self.P, ptr(self.tsort), self.npts, _lib.ints(self.grid_size),
+                                            _lib.ints(self.wrap), self.width, _lib.doubles(self.betas),
+                                            ptr(self.wsort), ptr(self.lbase), st))
             self.subgrid = int(L.mra_subgrid_points(D, self.P))
             self.max_coil_chunk = int(L.mra_max_coil_chunk(D, self.P))
         # The only host synchronisation of a plan: the number of work items, which
