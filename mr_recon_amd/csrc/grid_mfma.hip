@@ -96,8 +96,10 @@ __device__ __forceinline__ float take(v4f& a, bool act) {
   return v;
 }
 
-// Stores of an item's subgrids: byte offsets from the item's slot, out of range (dropped by the
-// hardware's bounds check) for lanes without a value and for coils past the last.
+// Stores of an item's subgrids: byte offset lane_off + off from the item's slot. The hardware
+// drops a store whose lane_off is past the nc subgrids of the slot; `off` is no part of that
+// check, so it only moves inside one subgrid, and lane_off carries the coil (past the range for
+// coils past the last) or kNoLane (lanes without a value).
 struct SlotStore {
   __amdgpu_buffer_rsrc_t rsrc;
   __device__ __forceinline__ SlotStore(float2* dst, int nbytes)
@@ -341,7 +343,7 @@ __device__ __forceinline__ void retire_row(const M& m, v4f (&acc)[M::NW][M::NB],
       const float a = 2 * k < M::NW ? v[2 * k < M::NW ? 2 * k : 0] : 0.f;
       const float lo = (2 * k >= 1 && 2 * k - 1 < M::NW) ? r[2 * k >= 1 ? (2 * k - 1) % M::NW : 0] : 0.f;
       const float hi = 2 * k + 1 < M::NW ? r[(2 * k + 1) % M::NW] : 0.f;
-      out.put(a + (x < 8 ? lo : hi), k + 1 < M::NK ? l0 : l1, (row * M::SUB + 16 * k + nb * M::SUBN) * 8);
+      out.put(a + (x < 8 ? lo : hi), (k + 1 < M::NK ? l0 : l1) + nb * (M::SUBN * 8), (row * M::SUB + 16 * k) * 8);
     }
   }
 }
@@ -549,17 +551,17 @@ __device__ __forceinline__ void retire_plane(const M& m, v4f (&acc)[M::NH][M::NB
   for (int nb = 0; nb < M::NB; ++nb)
 #pragma unroll
     for (int b = 0; b < M::NBLK; ++b) {
-      const int at = (pl * M::PP + b * M::RP * M::SUB + nb * M::SUBN) * 8;
+      const int at = (pl * M::PP + b * M::RP * M::SUB) * 8, coil = nb * (M::SUBN * 8);
       const bool end = b + 1 == M::NBLK;
       if constexpr (M::NARROW) {
         // columns 0..3 window 0, 4..7 both, 8..11 window 1
         const float v0 = take<E>(acc[0][b][nb], act), v1 = take<E>(acc[1][b][nb], act);
         const float s1 = shift4(v1);
-        out.put(x >= 4 ? v0 + s1 : v0, end ? l0e : l0, at);
-        out.put(v1, end ? l1e : l1, at);
+        out.put(x >= 4 ? v0 + s1 : v0, (end ? l0e : l0) + coil, at);
+        out.put(v1, (end ? l1e : l1) + coil, at);
       } else {
         const float v = take<E>(acc[0][b][nb], act);
-        out.put(v, end ? l0e : l0, at);
+        out.put(v, (end ? l0e : l0) + coil, at);
       }
     }
 }
