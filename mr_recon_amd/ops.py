@@ -394,6 +394,8 @@ def toeplitz_normal(x: torch.Tensor, im_size, grid_size, smaps: torch.Tensor, ke
     G = tuple(int(g) for g in grid_size)
     x = _c64(x, "x").reshape(1, *im_size)
     smaps = _c64(smaps, "smaps")
+    if tuple(smaps.shape[-D:]) != tuple(im_size):
+        raise ValueError("maps must have the image shape")
     C = int(math.prod(smaps.shape[:-D]))
     compiled = D >= 2 and fused_supported(G)
     if not compiled and (D < 2 or tuple(kern_unshifted.shape) != G or not fused_any_supported(G)):
