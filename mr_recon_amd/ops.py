@@ -342,6 +342,8 @@ def ifft_crop(grid: torch.Tensor, im_size, grid_size, nx: int, smaps: torch.Tens
     D = len(im_size)
     G = tuple(int(g) for g in grid_size)
     compiled = fused_supported(G)
+    if not compiled and grid.numel() % math.prod(G):
+        raise ValueError(f"ifft_crop: {grid.numel()} values are not whole grids of shape {G}")
     if not compiled and (coil_off is not None or not grid.is_contiguous() or not fused_any_supported(G)):
         if coil_off is not None:
             raise ValueError("ifft_crop: batched reduction needs a grid with an LDS FFT plan")

@@ -17,3 +17,12 @@ def test_toeplitz_refuses_maps_of_another_shape(N, G, trailing):
     x, kern = torch.zeros(N, dtype=torch.complex64), torch.zeros(G, dtype=torch.complex64)
     with pytest.raises(ValueError, match="image shape"):
         ops.toeplitz_normal(x, N, G, torch.zeros((3, *trailing(N)), dtype=torch.complex64), kern)
+
+
+@pytest.mark.parametrize("N,G", GRIDS[1:])
+@pytest.mark.parametrize("n", [lambda g: g + 1, lambda g: 2 * g - 1])
+def test_ifft_crop_refuses_parts_of_a_grid(N, G, n):
+    """Values behind the last whole grid are a mistake of the caller's, not to be dropped."""
+    grid = torch.zeros(n(G[0] * G[1]), dtype=torch.complex64)
+    with pytest.raises(ValueError, match="whole grids"):
+        ops.ifft_crop(grid, N, G, 1)
