@@ -62,7 +62,7 @@ class _LdsFFT:
             if arr is None:
                 tabs = []
                 for L in shape:
-                    host = torch.empty(2 * L, dtype=torch.float32)
+                    host = torch.empty(2 * L, dtype=torch.float32, device="cpu")  # whatever the default device
                     check(lib().mra_fft_lds_twiddles(L, ctypes.cast(host.data_ptr(), ctypes.POINTER(ctypes.c_float))))
                     tabs.append(host.to(device))
                 arr = (tabs, (ctypes.c_void_p * len(shape))(*[t.data_ptr() for t in tabs]))
@@ -90,7 +90,8 @@ class _AnyFFT:
                 for L in shape:
                     t = self._tab.get((device.index, L))
                     if t is None:
-                        host = torch.empty(2 * int(lib().mra_fft_any_table_len(L)), dtype=torch.float32)
+                        n = 2 * int(lib().mra_fft_any_table_len(L))
+                        host = torch.empty(n, dtype=torch.float32, device="cpu")  # whatever the default device
                         check(lib().mra_fft_any_table(L, ctypes.cast(host.data_ptr(), ctypes.POINTER(ctypes.c_float))))
                         t = self._tab[(device.index, L)] = host.to(device)
                     tabs.append(t)

@@ -26,3 +26,21 @@ def test_ifft_crop_refuses_parts_of_a_grid(N, G, n):
     grid = torch.zeros(n(G[0] * G[1]), dtype=torch.complex64)
     with pytest.raises(ValueError, match="whole grids"):
         ops.ifft_crop(grid, N, G, 1)
+
+
+@pytest.mark.parametrize("tables,L,values", [("_any_fft", 76, 76), ("_any_fft", 97, 97 + 2 * 195), ("_lds_fft", 64, 64)])
+def test_tables_under_another_default_device(tables, L, values):
+    """The library fills the tables through a host address, whatever device new tensors go to by
+    default; the first L values are the length's roots (chirp tables start with those of their M)."""
+    from mr_recon_amd import gridfft
+
+    own = type(getattr(gridfft, tables))()
+    with torch.device("meta"):
+        own.tables(torch.device("cpu"), (L,))
+    tab = (own._arr if tables == "_any_fft" else own._tw)[(None, (L,))][0][0]
+    assert tab.device.type == "cpu" and tab.numel() == 2 * values
+    M = 195 if values > L else L
+    got = torch.view_as_complex(tab.view(-1, 2))[:M].to(torch.complex128)
+    m = torch.arange(M, dtype=torch.float64)
+    want = torch.polar(torch.ones(M, dtype=torch.float64), -2 * torch.pi * m / M)
+    assert float((got - want).abs().max()) < 1e-7
