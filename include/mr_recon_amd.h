@@ -185,6 +185,7 @@ int mra_toeplitz_fused(int ndim, const int* N, const int* G, const int* center, 
  * mra_fft_any_table(G[d]), mra_fft_any_table_len(G[d]) complex values. One image batch, no
  * per-problem indexing; mra_fft_crop_adjoint_any takes nx * ns grids. */
 int mra_fft_any_supported(int ndim, const int* G);
+int mra_fft_any_shape(int L, int* shape); /* 16 ints: M, threads, transforms, kind, LDS bytes, passes, radices */
 long long mra_fft_any_table_len(int L);
 int mra_fft_any_table(int L, float* host);
 int mra_fft_pad_forward_any(int ndim, const int* N, const int* G, const int* center, const void* x, long long x_stride,

@@ -75,6 +75,7 @@ SIGNATURES = {
                                   C.POINTER(_vp), _vp]),
     "mra_toeplitz_fused": (_i, [_i, _ip, _ip, _ip, _vp, _vp, _ll, _ll, _vp, _vp, _i, _vp, C.POINTER(_vp), _vp]),
     "mra_fft_any_supported": (_i, [_i, _ip]),
+    "mra_fft_any_shape": (_i, [_i, _ip]),
     "mra_fft_any_table_len": (_ll, [_i]),
     "mra_fft_any_table": (_i, [_i, _fp]),
     "mra_fft_pad_forward_any": (_i, [_i, _ip, _ip, _ip, _vp, _ll, _vp, _ll, _ll, _ll, _vp, _f, _vp, C.POINTER(_vp), _vp]),

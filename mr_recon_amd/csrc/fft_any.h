@@ -165,6 +165,12 @@ inline const AnyPlan* any_plan(int L) {
 // What a kernel is compiled for: direct passes up to radix 16, the chirp-z form over them, and
 // direct passes with radix 17 or 19 (whose registers halve the blocks of a CU at 1024 threads).
 enum AnyKind { kDirect = 0, kChirp = 1, kPrime = 2 };
+inline AnyKind any_kind(const AnyPlan& p) {
+  if (p.M != p.L) return kChirp;
+  for (int i = 0; i < p.npass; ++i)
+    if (p.radix[i] > 16) return kPrime;
+  return kDirect;
+}
 
 template <int TPB, int NT>
 struct Any {
@@ -262,11 +268,10 @@ template <class F>
 int with_any(const AnyPlan& p, F&& f) {
   using std::integral_constant;
   const AnyShape s = any_shape(p);
-  bool prime = false;
-  for (int i = 0; i < p.npass; ++i) prime = prime || p.radix[i] > 16;
+  const AnyKind kind = any_kind(p);
   auto go = [&](auto TPB, auto NT) {
-    if (p.M != p.L) return f(TPB, NT, integral_constant<int, kChirp>{});
-    return prime ? f(TPB, NT, integral_constant<int, kPrime>{}) : f(TPB, NT, integral_constant<int, kDirect>{});
+    if (kind == kChirp) return f(TPB, NT, integral_constant<int, kChirp>{});
+    return kind == kPrime ? f(TPB, NT, integral_constant<int, kPrime>{}) : f(TPB, NT, integral_constant<int, kDirect>{});
   };
   if (s.nt == 8) return go(integral_constant<int, 1024>{}, integral_constant<int, 8>{});
   if (s.tpb == 256) return go(integral_constant<int, 256>{}, integral_constant<int, 16>{});

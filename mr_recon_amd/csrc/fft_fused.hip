@@ -812,6 +812,19 @@ int mra_fft_any_supported(int ndim, const int* G) {
   return 1;
 }
 
+// How the *_any entry points run length L: shape = {M (the length transformed: L, or the chirp-z
+// form's convolution), threads of a block, transforms of a block, kind (0 direct, 1 chirp-z,
+// 2 direct with radix 17 or 19), dynamic LDS bytes, passes, radix of each pass}, 16 ints.
+int mra_fft_any_shape(int L, int* shape) {
+  MRA_TRY_BEGIN
+  const fft::AnyPlan* p = fft::any_plan(L);
+  if (!p) MRA_FAIL("fft: length outside 2..640");
+  const fft::AnyShape s = fft::any_shape(*p);
+  const int head[] = {p->M, s.tpb, s.nt, fft::any_kind(*p), (int)s.lds, p->npass};
+  for (int i = 0; i < 16; ++i) shape[i] = i < 6 ? head[i] : i - 6 < p->npass ? p->radix[i - 6] : 0;
+  MRA_TRY_END
+}
+
 // Device table of length L for the *_any entry points: complex values, and their contents
 // (host memory). For lengths with a compiled plan the first L values are mra_fft_lds_twiddles'.
 long long mra_fft_any_table_len(int L) {
