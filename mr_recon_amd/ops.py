@@ -121,7 +121,8 @@ def gridding_noalloc(ksp: torch.Tensor, plan: SamplePlan, out: torch.Tensor, dcf
                      out_scale: float = 1.0, accumulate: bool = False) -> torch.Tensor:
     """``gridding`` without any device allocation: the phase-1 subgrids go to the library's
     static scratch (``mra_grid_noalloc``), so the call can run under HIP graph capture. Raises
-    when the plan needs more scratch than that array holds. Calls that overlap on one GPU
+    when the plan needs more scratch than that array holds (plans cut their samples into longer
+    work items where that lets more batch entries fit). Calls that overlap on one GPU
     share the array and must not run concurrently."""
     import ctypes
 

@@ -42,13 +42,30 @@ def binning_chunk(npts: int, ntiles: int, tile: int, ndim: int) -> int:
     return min(c, 4096)
 
 
-def default_samples_per_item(npts: int, ndim: int = 2) -> int:
-    """Work-item size: about a thousand items per trajectory, 256..8192 samples each; in 3D at
-    most 2560, so that the tiles of the k-space centre do not end a launch alone (5.12 M samples,
-    32 coils: gridding 3.62 -> 3.47 ms against 5120 samples an item)."""
+def item_lengths(npts: int, ndim: int = 2) -> tuple:
+    """Work-item sizes to choose from, the preferred one first: about a thousand items per
+    trajectory, 256..8192 samples each; in 3D at most 2560, so that the tiles of the k-space centre
+    do not end a launch alone (gridding to images of a 128^3 kooshball of 5.12 M samples, 2560 /
+    5120 samples an item: 32 coils 4.37 / 4.53 ms, 16 coils 2.34 / 2.54, 4 coils 0.87 / 1.08), with
+    the uncapped size second."""
     s = -(-npts // 1024)
-    s = -(-s // 256) * 256
-    return int(min(max(s, 256), 2560 if ndim == 3 else 8192))
+    s = min(max(-(-s // 256) * 256, 256), 8192)
+    return (2560, s) if ndim == 3 and s > 2560 else (s,)
+
+
+def default_samples_per_item(npts: int, ndim: int = 2) -> int:
+    """Preferred work-item size (``item_lengths``)."""
+    return item_lengths(npts, ndim)[0]
+
+
+def choose_item_length(nitems, subgrid: int, limit: int) -> int:
+    """Index of the work-item size a plan takes, of those that cut it into ``nitems`` items
+    (preferred size first) with subgrids of ``subgrid`` points: the first one, unless the
+    no-allocation gridding scratch (``limit`` bytes) holds more batch entries with a later one.
+    Shorter items mean more partial subgrids, and a call that fits must not stop fitting (14 M
+    samples on an 80^3 grid, one entry: 81 MB with items of 2560 samples, 30 MB with 8192)."""
+    entries = [limit // (n * subgrid * 8) for n in nitems]
+    return entries.index(max(entries))
 
 
 def batch_samples_per_item(npts: int) -> int:
@@ -126,8 +143,8 @@ class SamplePlan:
             pass
         self.ntile = [(g + self.tile - 1) // self.tile for g in self.grid_size]
         self.ntiles = int(math.prod(self.ntile))
-        self.S = int(samples_per_item or default_samples_per_item(self.npts, D))
-        if self.S < 1:
+        lengths = (int(samples_per_item),) if samples_per_item else item_lengths(self.npts, D)
+        if lengths[0] < 1:
             raise ValueError("samples_per_item must be positive")
         self.wrap = tuple(int(w) for w in (wrap if wrap is not None else (0,) * D))
 
@@ -149,15 +166,16 @@ class SamplePlan:
         check(L.mra_bin_build(D, ptr(flat), self.npts, _lib.ints(self.grid_size), sc, sh, int(apply),
                               self.width, self.tile, _lib.ints(self.wrap), chunk, ptr(work), ptr(self.tsort),
                               ptr(self.perm), ptr(self.tile_start), st))
-        self.max_items = nkeys + (self.npts + self.S - 1) // self.S
-        self.items = torch.empty((self.max_items, 4), dtype=torch.int32, device=dev)
         nitems_ws = torch.empty(nkeys + 1, dtype=torch.int32, device=dev)
-        item_off = torch.empty(nkeys + 1, dtype=torch.int32, device=dev)
         scan_ws2 = torch.empty(L.mra_scan_workspace(nkeys + 1), dtype=torch.int32, device=dev)
-        check(L.mra_bin_items(ptr(self.tile_start), self.ntiles, self.S, 0, ptr(nitems_ws), ptr(item_off),
-                              ptr(scan_ws2), ptr(self.items), self.max_items, st))
-        # item_off[t] is the first work item of tile t (t = ntiles: non-finite samples)
-        self.tile_items = item_off
+        cuts = []  # per work-item size: the items, and the first of each tile (tile ntiles: non-finite samples)
+        for S in lengths:
+            max_items = nkeys + (self.npts + S - 1) // S
+            items = torch.empty((max_items, 4), dtype=torch.int32, device=dev)
+            item_off = torch.empty(nkeys + 1, dtype=torch.int32, device=dev)
+            check(L.mra_bin_items(ptr(self.tile_start), self.ntiles, S, 0, ptr(nitems_ws), ptr(item_off),
+                                  ptr(scan_ws2), ptr(items), max_items, st))
+            cuts.append((S, items, item_off))
         # KB weights (D x P per sorted sample) and subgrid offsets, once per trajectory
         self.wsort = torch.empty(self.npts * D * self.P, dtype=torch.float32, device=dev)
         self.lbase = torch.empty(self.npts, dtype=torch.int32, device=dev)
@@ -169,10 +187,17 @@ class SamplePlan:
             self.max_coil_chunk = int(L.mra_max_coil_chunk(D, self.P))
         # The only host synchronisation of a plan: the number of work items, which
         # sizes the launches and the gridding scratch.
-        self.nitems = int(item_off[nkeys].item())
+        if len(cuts) == 1:
+            nitems = [int(cuts[0][2][nkeys].item())]
+        else:
+            nitems = torch.stack([off[nkeys] for _, _, off in cuts]).tolist()
+        i = choose_item_length(nitems, self.subgrid, int(L.mra_grid_noalloc_max_bytes()))
+        self.nitems = nitems[i]
+        self.S, self.items, self.tile_items = cuts[i]
+        self.max_items = self.items.shape[0]
         # The workspaces go back to the caching allocator here; PyTorch only
         # hands them out again to work ordered after these kernels on this stream.
-        del work, nitems_ws, scan_ws2, flat
+        del work, nitems_ws, scan_ws2, flat, cuts, items, item_off
         self._geoms: dict[GeomKey, torch.Tensor] = {}
 
     def coil_chunk(self, nbatch: int) -> int:

@@ -1,0 +1,27 @@
+"""The rules for the length of a work item (no GPU)."""
+
+import pytest
+
+from mr_recon_amd import plan
+
+
+@pytest.mark.parametrize("npts,ndim,want", [(1, 2, (256,)), (262144, 3, (256,)), (262145, 3, (512,)),
+                                            (2_621_440, 3, (2560,)), (2_621_441, 3, (2560, 2816)),
+                                            (5_120_000, 3, (2560, 5120)), (20_000_000, 3, (2560, 8192)),
+                                            (20_000_000, 2, (8192,)), (5_120_000, 1, (5120,))])
+def test_lengths(npts, ndim, want):
+    assert plan.item_lengths(npts, ndim) == want
+    assert plan.default_samples_per_item(npts, ndim) == want[0]
+
+
+@pytest.mark.parametrize("nitems", [(5898, 2144), (3700, 1500), (5755, 5297), (4800, 4700), (1000, 400), (9000, 4000)])
+@pytest.mark.parametrize("P", [4, 5, 7])
+def test_no_batch_that_fitted_is_refused(nitems, P):
+    """The no-allocation scratch holds as many batch entries as with the longest items."""
+    limit, sub = (64 << 20) - 256, (7 + P) ** 3
+    i = plan.choose_item_length(nitems, sub, limit)
+    for batch in range(1, 70):
+        if nitems[-1] * batch * sub * 8 <= limit:
+            assert nitems[i] * batch * sub * 8 <= limit
+    if limit // (nitems[0] * sub * 8) == limit // (nitems[1] * sub * 8):
+        assert i == 0  # the preferred size where it refuses nothing
