@@ -155,7 +155,7 @@ def density_compensation(trj: torch.Tensor, im_size: tuple, num_iters: Optional[
     exists in the reference (its other branches are commented out).
     """
     from . import ops
-    from .plan import SamplePlan, default_samples_per_item
+    from .plan import SamplePlan, dcf_samples_per_item
 
     method = method.lower()
     if method != "sigpy":
@@ -168,10 +168,8 @@ def density_compensation(trj: torch.Tensor, im_size: tuple, num_iters: Optional[
     if num_iters is None or num_iters < 0:
         raise ValueError("num_iters must be a non-negative integer")
     coords = trj.reshape(-1, D).to(torch.float32).contiguous()
-    # half the usual items' length: one batch entry leaves one wave to an item (96^3, 1.5 M
-    # samples, an iteration: 209 us, 182 at half, 183 at a quarter)
     plan = SamplePlan(coords, im_size, PIPE_MENON_WIDTH, PIPE_MENON_BETA,
-                      samples_per_item=max(256, default_samples_per_item(coords.shape[0], D) // 2))
+                      samples_per_item=dcf_samples_per_item(coords.shape[0], D))
     M = plan.npts
     dev = trj.device
     st = stream_ptr(dev)

@@ -75,6 +75,16 @@ def batch_samples_per_item(npts: int) -> int:
     return min(default_samples_per_item(npts // 2), 1024)
 
 
+def dcf_samples_per_item(npts: int, ndim: int) -> int:
+    """Work-item size of density compensation, whose one batch entry leaves one wave to an item:
+    half the usual length, so that the launch does not end on its longest items, but not below 512
+    samples, where the partial subgrids cost more than that (one iteration, us, at the usual length
+    / half / a quarter: 96^3, 1.5 M samples: 178 / 151 / 169; 128^3, 5.1 M: 542 at 5120, 378 at 1280;
+    256^2, 2 M: 140 / 128 / 152; at 512 / 256: 64^3, 0.38 M: 78 / 85; 256^2, 0.41 M: 53 / 62)."""
+    s = default_samples_per_item(npts, ndim)
+    return max(s // 2, min(s, 512))
+
+
 def kernel_points(width: float) -> int:
     """Grid points per dimension a KB patch of width ``width`` can touch."""
     return int(math.floor(float(width))) + 1

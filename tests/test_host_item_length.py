@@ -25,3 +25,11 @@ def test_no_batch_that_fitted_is_refused(nitems, P):
             assert nitems[i] * batch * sub * 8 <= limit
     if limit // (nitems[0] * sub * 8) == limit // (nitems[1] * sub * 8):
         assert i == 0  # the preferred size where it refuses nothing
+
+
+@pytest.mark.parametrize("npts,ndim,want", [(1000, 2, 256), (262144, 3, 256), (288_000, 3, 512), (409_600, 2, 512),
+                                            (640_000, 3, 512), (960_000, 3, 512), (1_536_000, 3, 768),
+                                            (5_120_000, 3, 1280), (8_192_000, 2, 4096)])
+def test_dcf_length(npts, ndim, want):
+    """Half the usual length, but items of 512 samples are not halved."""
+    assert plan.dcf_samples_per_item(npts, ndim) == want
