@@ -115,14 +115,14 @@ class BatchedSense:
         if tile == "auto":
             tile, self.tile_times = self._tune_tile(problems, oversamp, width, samples_per_item)
         self.problems = list(problems)
-        if samples_per_item is None:
-            samples_per_item = batch_samples_per_item(sum(pr.trj.numel() // 2 for pr in self.problems))
         sizes = {}
         for i, pr in enumerate(self.problems):
             _lib.require_device(pr.trj, pr.mps)
             if pr.mps.ndim != 3 or pr.mps.shape[1] != pr.mps.shape[2]:
                 raise ValueError("batched problems are 2D with square images: mps (C, N, N)")
             sizes.setdefault(int(pr.mps.shape[1]), []).append(i)
+        if samples_per_item is None:
+            samples_per_item = batch_samples_per_item((pr.trj.numel() // 2, pr.mps.shape[0]) for pr in self.problems)
         self.groups = [_Group(idx, self.problems, N, oversamp, width, samples_per_item, tile)
                        for N, idx in sorted(sizes.items())]
         g0 = self.groups[0]

@@ -68,11 +68,20 @@ def choose_item_length(nitems, subgrid: int, limit: int) -> int:
     return entries.index(max(entries))
 
 
-def batch_samples_per_item(npts: int) -> int:
-    """Work-item size of problems that share their launches, ``npts`` samples in all: other
-    problems' items fill the device, so an item may be longer, which saves partial subgrids
-    (24 problems of 20..130 k samples: 14.5 ms at 256 samples, 12.8 at 512, 12.5 at 1024)."""
-    return min(default_samples_per_item(npts // 2), 1024)
+def batch_samples_per_item(sizes) -> int:
+    """Work-item size of problems that share their launches, ``sizes`` their (samples, coils):
+    other problems' items fill the device, so an item may be longer, which saves partial subgrids,
+    as long as about 4096 waves (of four coils) are left. Normal operator of a batch, us at 256 /
+    512 / 1024 samples an item:
+      24 problems x 25.6 k x 8 coils   191 /  202 /  229     24 x 25.6 k x 32       660 / 609 / 607
+      24 x 51 k x 4                    347 /  360 /  388     16 x 131 k x 16       1068 / 928 / 947
+      12 x 102 k x 8                   391 /  369 /  396     24 x 410 k x 8        1545 / 1244 / 1156
+    and 24 of 20..130 k x 8..32 with 8 solver steps 14.5 / 12.8 / 12.5 ms; 2048 samples were slower
+    than 1024 up to 8 M samples a problem (8 x 2 M x 8: 1355 / 1395 us)."""
+    sizes = list(sizes)
+    waves = sum(n * -(-c // 4) for n, c in sizes)
+    fill = (waves // 4096 + 128) // 256 * 256
+    return min(default_samples_per_item(sum(n for n, _ in sizes) // 2), 1024, max(fill, 256))
 
 
 def dcf_samples_per_item(npts: int, ndim: int) -> int:

@@ -33,3 +33,12 @@ def test_no_batch_that_fitted_is_refused(nitems, P):
 def test_dcf_length(npts, ndim, want):
     """Half the usual length, but items of 512 samples are not halved."""
     assert plan.dcf_samples_per_item(npts, ndim) == want
+
+
+@pytest.mark.parametrize("n,npts,coils,want", [
+    (64, 7680, 4, 256), (24, 25_600, 8, 256), (24, 51_200, 4, 256), (12, 49_920, 8, 256), (4, 102_400, 8, 256),
+    (24, 25_600, 16, 512), (24, 40_960, 8, 512), (12, 102_400, 8, 512), (2, 512_000, 8, 512), (12, 49_920, 32, 512),
+    (32, 51_200, 8, 768), (24, 76_800, 12, 1024), (16, 131_072, 16, 1024), (24, 409_600, 8, 1024), (0, 1, 1, 256)])
+def test_batch_length(n, npts, coils, want):
+    """Longer items only where enough waves are left to fill the device."""
+    assert plan.batch_samples_per_item([(npts, coils)] * n) == want
