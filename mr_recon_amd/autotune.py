@@ -8,12 +8,15 @@ blocks many, large ones cut the subgrid halo (a 16 x 16 tile's subgrid at P = 5 
 1.56x its area, a 32 x 32 one's 1.27x) and with it the gridding scratch.
 ``tune_work`` times interp + gridding on the caller's own trajectory for every
 candidate pair and keeps the fastest; results are cached in a JSON table keyed by
-(ndim, kernel points, grid size, samples/tile bucket, batch bucket, tile choice)
-so later plans of the same class skip the search.
+(built kernels, device, ndim, kernel points, grid size, samples/tile bucket, batch
+bucket, tile choice) so later plans of the same class skip the search. A choice timed
+on other kernels or another device is not used.
 """
 
 from __future__ import annotations
 
+import functools
+import hashlib
 import json
 import math
 import os
@@ -59,6 +62,16 @@ def tune_key(ndim: int, width: float, grid_size, npts: int, nbatch: int) -> str:
             f"s{1 << int(math.log2(dens))}-b{1 << int(math.log2(max(1, nbatch)))}")
 
 
+@functools.lru_cache(maxsize=None)
+def _kernels() -> str:
+    """The built kernels: a digest of the library (11 MB, a few ms once per process)."""
+    return hashlib.blake2b(_lib.LIB_PATH.read_bytes(), digest_size=6).hexdigest()
+
+
+def _device(device: torch.device) -> str:
+    return torch.cuda.get_device_properties(device).gcnArchName.split(":")[0] if device.type == "cuda" else device.type
+
+
 def _time(fn, reps: int = 3) -> float:
     fn()
     torch.cuda.synchronize()
@@ -82,7 +95,7 @@ def tune_work(coords: torch.Tensor, grid_size, width: float, beta: float, nbatch
     L = _lib.lib()
     tiles = tuple(tiles) if tiles is not None else (TILES[D] if tune_tile else (int(L.mra_default_tile(D)),))
     samples = tuple(samples) if samples is not None else CANDIDATES
-    key = tune_key(D, width, grid_size, M, nbatch) + "-t" + "_".join(map(str, tiles)) + \
+    key = f"{_kernels()}-{_device(coords.device)}-" + tune_key(D, width, grid_size, M, nbatch) + "-t" + "_".join(map(str, tiles)) + \
         "-s" + "_".join(map(str, samples))
     with _lock:
         table = _load()
