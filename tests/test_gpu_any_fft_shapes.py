@@ -46,3 +46,18 @@ def test_launch_shapes(dev, N, G, ns):
     want = _ref_crop(spec, N, G, cen, smaps, one, 1.0, True)
     got = ops.toeplitz_normal(x[0], N, G, smaps, kern)
     assert rel_l2(got, want.to(got.dtype)) < TOL
+
+
+@pytest.mark.parametrize("L,tol", [(88, 1.2e-7), (90, 1.2e-7), (136, 1.2e-7), (152, 1.2e-7), (340, 1.2e-7),
+                                   (97, 3e-7), (211, 3e-7), (467, 3e-7)])
+def test_rows_against_64_bits(dev, L, tol):
+    """Relative L2 error of rows of random values. A rounding to 32 bits adds about 0.3e-7; a direct
+    transform of two or three passes rounds a value some ten times, in its twiddle products and
+    sums (radix 17 and 19 sum in 64 bits); the chirp-z form is two transforms of 2 L points and three
+    products."""
+    from mr_recon_amd import ops
+
+    x = _rand((512, L), L, dev)
+    got = ops.pad_fft(x, (L,), (L,), center=(0,)).to(torch.complex128)
+    want = torch.fft.fft(x.to(torch.complex128), dim=-1)
+    assert float((got - want).norm() / want.norm()) < tol
