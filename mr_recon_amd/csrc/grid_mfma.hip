@@ -24,7 +24,11 @@
 //       P >= 6: row pairs (2 x 8 corners); a block is one row x 16 columns, P + 1 blocks.
 //   R = 4 where the samples reach at most 4 planes, else 8. With P = 5 that holds for every
 //   sample but those whose t - w/2 falls on a grid integer (w = 4: the k-space centre of radial
-//   trajectories, and a few by chance). An item with one of them takes R = 8.
+//   trajectories, and one in some 60 000 by rounding). An item with one of them takes R = 8: in 2D
+//   with twice the blocks for the same coils, in 3D, where those would cost a third of the waves,
+//   for half the coils at a time. A 2D launch lasts as long as such items: at half the coils they
+//   took twice the chain (40 us in the 131 k x 16 case below, 878 us against 835 for 2 M radial
+//   samples x 32).
 //
 // Values that would not stay inside the patch: a block also multiplies a sample's zero weights
 // outside its patch, and 0 * inf = nan. Samples with a k-space value (times dcf) or weights that
@@ -36,9 +40,9 @@
 // matrix rate in the 3D 128^3 case, 2 waves per SIMD; skipping all but one of a group's products
 // takes 11 % off, skipping the gathers 20 %). Phase 1 before (2D: per-lane LDS read-modify-
 // writes; 3D: products per cell added to an LDS plane ring) and now, MI355X:
-//   3D 5.12 M samples x 32 coils, P 5   4.88 -> 2.58 ms     0.76 M x 7, P 7   1.00 -> 0.34 ms
-//   3D 1.5 M samples x 1, P 5            155 -> 114 us      2D 131 k x 16, P 5  80 -> 37 us
-//   2D 131 k samples x 16, P 7            94 -> 36 us       2D 4096 x 1, P 7    83 -> 16 us
+//   3D 5.12 M samples x 32 coils, P 5   4.88 -> 2.30 ms     0.76 M x 7, P 7   1.00 -> 0.33 ms
+//   3D 1.5 M samples x 1, P 5            155 -> 110 us      2D 131 k x 16, P 5  80 -> 30 us
+//   2D 131 k samples x 16, P 7            94 -> 34 us       2D 4096 x 1, P 7    83 -> 15 us
 #include <type_traits>
 
 #include "grid_mfma.h"
@@ -277,43 +281,35 @@ struct Groups {
   __device__ __forceinline__ int at(int g) const { return g < n ? __builtin_amdgcn_readlane(word, g) : kEnd; }
 };
 
-// Ring of a wave: R slots times the (coil, re/im) components of 16 / R rows, NB matrix blocks.
-// Component 2c + re/im of block nb is coil c NB + nb, so that a wave which goes over from 4 to 8
-// slots (P = 5) finds the first NB coils where they were.
-template <int P, int NB>
+// Ring of a wave: R slots (4 where the samples reach at most 4 planes, else 8) times the (coil,
+// re/im) components of 16 / R rows, NB matrix blocks. Component 2c + re/im of block nb is coil
+// c NB + nb.
+template <int P, int NB, int R>
 struct Ring {
-  static constexpr int R0 = P <= 5 ? 4 : 8;    // slots an item starts with
-  static constexpr bool DUAL = P == 5;         // 8 slots for items that reach the fifth plane
-  static constexpr int ZN = DUAL ? 8 : R0;     // dim-0 weights staged
-  static constexpr int NC = NB * 8 / R0;       // coils per wave (with R0 slots)
-  static constexpr int YC = 16 / R0;           // components staged
-  int r;
-  __device__ __forceinline__ explicit Ring(int slots) : r(DUAL ? slots : R0) {}
-  __device__ __forceinline__ int slots() const { return DUAL ? r : R0; }
-  __device__ __forceinline__ int slot(int row16) const { return row16 & (slots() - 1); }
-  __device__ __forceinline__ int comp(int row16) const { return slots() == 4 ? row16 >> 2 : row16 >> 3; }
+  static_assert((R == 4 && P <= 5) || R == 8, "ring");
+  static constexpr int NC = NB * 8 / R;        // coils of a wave
+  static constexpr int YC = 16 / R;            // components staged
+  static __device__ __forceinline__ int slot(int row16) { return row16 & (R - 1); }
+  static __device__ __forceinline__ int comp(int row16) { return row16 / R; }
   // result layout: lane group q holds rows 4q .. 4q+3, so element e is slot e (4 slots) or
   // 4 (q mod 2) + e (8 slots) of component:
-  __device__ __forceinline__ int comp_of_group(int q) const { return slots() == 4 ? q : q >> 1; }
-  __device__ __forceinline__ bool holds(int q, int plane) const {
-    return slots() == 4 || (q & 1) == ((plane >> 2) & 1);
-  }
+  static __device__ __forceinline__ int comp_of_group(int q) { return R == 4 ? q : q >> 1; }
+  static __device__ __forceinline__ bool holds(int q, int plane) { return R == 4 || (q & 1) == ((plane >> 2) & 1); }
 };
+constexpr int ring_slots(int P) { return P <= 5 ? 4 : 8; }  // of items that miss the fifth plane
 
 // ---- 2D -------------------------------------------------------------------------------------
 
-template <int P_, int T_, int NB_>
-struct Rows2 : Ring<P_, NB_> {
-  using Ring<P_, NB_>::Ring;
-  using Ring<P_, NB_>::ZN;
-  using Ring<P_, NB_>::YC;
+template <int P_, int T_, int NB_, int R>
+struct Rows2 : Ring<P_, NB_, R> {
+  using Ring<P_, NB_, R>::YC;
   static constexpr int P = P_, T = T_, NB = NB_;
   static constexpr int SUB = T + P - 1, SUBN = SUB * SUB;
   static constexpr int NW = T / 8;             // windows of 8 corners per row
   static constexpr int NK = (SUB + 15) / 16;   // 16-column stores per subgrid row
-  // stage record of a sample (floats): 16 dim-1 weights, ZN dim-0 weights, the k-space values by
+  // stage record of a sample (floats): 16 dim-1 weights, R dim-0 weights, the k-space values by
   // component; padded so that 16-byte accesses of consecutive lanes spread over all banks
-  static constexpr int ZO = 16, YO = ZO + ZN;
+  static constexpr int ZN = R, ZO = 16, YO = ZO + ZN;
   static constexpr int RS = (YO + YC * NB) % 8 == 4 ? YO + YC * NB : (YO + YC * NB + 8) / 8 * 8 - 4;
   static_assert(P <= 8 && 7 + P <= 16 && SUB <= 8 * (NW + 1), "window");
 };
@@ -322,12 +318,12 @@ struct Rows2 : Ring<P_, NB_> {
 // and clear its slot. Columns 8w .. 8w+7 are the first half of window w plus the second half of
 // window w - 1.
 template <class M, int E>
-__device__ __forceinline__ void retire_row(const M& m, v4f (&acc)[M::NW][M::NB], int row, int lane,
+__device__ __forceinline__ void retire_row(v4f (&acc)[M::NW][M::NB], int row, int lane,
                                            const SlotStore& out) {
   const int x = lane & 15, q = lane >> 4;
-  const int comp = m.comp_of_group(q);
+  const int comp = M::comp_of_group(q);
   const int loff = ((comp >> 1) * M::NB * M::SUBN + x) * 8 + (comp & 1) * 4;
-  const bool act = m.holds(q, row);
+  const bool act = M::holds(q, row);
   const int l0 = act ? loff : kNoLane;
   const int l1 = M::SUB % 16 == 0 || x < M::SUB % 16 ? l0 : kNoLane;  // the last, partial 16 columns
 #pragma unroll
@@ -354,15 +350,14 @@ __device__ __forceinline__ void rows2_item(const float2* __restrict__ ksp, const
                                            const float* __restrict__ wsort, const int* __restrict__ lbase,
                                            const int* __restrict__ perm, const Geom* __restrict__ geoms,
                                            const Item* __restrict__ items, const Geom& g, const Item& it, int iidx,
-                                           int c0, int nc, int slots, float2* __restrict__ scratch, float* rec,
+                                           int c0, int nc, float2* __restrict__ scratch, float* rec,
                                            int* list) {
   constexpr int P = M::P, NB = M::NB, SUB = M::SUB;
-  const M m(slots);
   int lane = threadIdx.x;
   asm volatile("" : "+v"(lane));  // keeps lane terms from being carried across the caller's loop
   const int i16 = lane & 15;
   const int kq = (lane >> 4) ^ 2;  // the group's sample in this lane's K slot (their order is free)
-  const int zl = m.slot(i16), comp = m.comp(i16);  // this lane's A row
+  const int zl = M::slot(i16), comp = M::comp(i16);  // this lane's A row
   // byte offsets of this lane's operands from its group's first record
   const int off_w0 = (kq * M::RS + M::ZO) * 4, off_b = (kq * M::RS + i16) * 4;
   const int off_y = (kq * M::RS + M::YO + comp * NB) * 4;
@@ -395,7 +390,7 @@ __device__ __forceinline__ void rows2_item(const float2* __restrict__ ksp, const
   clear_planes(dst2, last, SUB, nc, M::SUB, M::SUBN, lane);
   int row = first;  // lowest row not yet stored
   auto retire_to = [&](int to) {
-    for (; row < to; ++row) with_element(row, [&](auto E) { retire_row<M, E.value>(m, acc, row, lane, out); });
+    for (; row < to; ++row) with_element(row, [&](auto E) { retire_row<M, E.value>(acc, row, lane, out); });
   };
 
   bool any_odd = false;
@@ -440,7 +435,7 @@ __device__ __forceinline__ void rows2_item(const float2* __restrict__ ksp, const
     } o;
     int g = 0, d = gr.at(0);  // the group whose operands are in `o`
     auto load_w0 = [&]() {  // this lane's ring slot holds patch plane zl - row (mod slots)
-      o.w0 = *(const float*)((const char*)rec + (d & 0xfff0) + off_w0 + m.slot(zl - row) * 4);
+      o.w0 = *(const float*)((const char*)rec + (d & 0xfff0) + off_w0 + M::slot(zl - row) * 4);
     };
     auto load = [&]() {
       const char* p = (const char*)rec + (d & 0xfff0);
@@ -490,8 +485,10 @@ __global__ __launch_bounds__(64) void grid_rows2d_kernel(const float2* __restric
                                                          const Geom* __restrict__ geoms,
                                                          const Item* __restrict__ items, int nitems, int nchunks,
                                                          float2* __restrict__ scratch) {
-  using M = Rows2<P, T, NB>;
-  __shared__ __attribute__((aligned(16))) float rec[kRows * M::RS];
+  constexpr int R = ring_slots(P);
+  using M = Rows2<P, T, NB, R>;
+  using W = Rows2<P, T, NB * (8 / R), 8>;  // the same coils with 8 slots
+  __shared__ __attribute__((aligned(16))) float rec[kRows * (P == 5 && W::RS > M::RS ? W::RS : M::RS)];
   __shared__ int list[kCh];
   int iidx, cc;
   item_of_block(blockIdx.x, nchunks, iidx, cc);
@@ -502,20 +499,20 @@ __global__ __launch_bounds__(64) void grid_rows2d_kernel(const float2* __restric
   const int c0 = cc * M::NC;
   if (c0 >= g.nbatch) return;
   const int nc = min(M::NC, g.nbatch - c0);
-  const int slots = M::DUAL && reaches_last_plane<2, P>(wsort, g, it) ? 8 : M::R0;
-  const int step = slots == M::R0 ? M::NC : NB;  // coils at a time
-  for (int c = 0; c < nc; c += step)
-    rows2_item<M>(ksp, dcf, wsort, lbase, perm, geoms, items, g, it, iidx, c0 + c, min(step, nc - c), slots, scratch, rec,
-               list);
+  if constexpr (P == 5) {
+    if (reaches_last_plane<2, P>(wsort, g, it)) {
+      rows2_item<W>(ksp, dcf, wsort, lbase, perm, geoms, items, g, it, iidx, c0, nc, scratch, rec, list);
+      return;
+    }
+  }
+  rows2_item<M>(ksp, dcf, wsort, lbase, perm, geoms, items, g, it, iidx, c0, nc, scratch, rec, list);
 }
 
 // ---- 3D -------------------------------------------------------------------------------------
 
-template <int P_, int NB_>
-struct Cells3 : Ring<P_, NB_> {
-  using Ring<P_, NB_>::Ring;
-  using Ring<P_, NB_>::ZN;
-  using Ring<P_, NB_>::YC;
+template <int P_, int NB_, int R>
+struct Cells3 : Ring<P_, NB_, R> {
+  using Ring<P_, NB_, R>::YC;
   static constexpr int P = P_, NB = NB_;
   static constexpr int T = 8, SUB = T + P - 1, PP = SUB * SUB, SUBN = SUB * PP;
   static constexpr bool NARROW = P <= 5;              // blocks of 2 rows x 8 columns, else 1 x 16
@@ -524,24 +521,24 @@ struct Cells3 : Ring<P_, NB_> {
   static constexpr int NH = NARROW ? 2 : 1;           // column windows (offset 4 apart)
   static constexpr int NBB = NARROW ? (P + 2) / 2 : P + 1;    // blocks a cell / row pair reaches
   static constexpr int NBLK = 6 / RP + NBB;           // blocks per plane and window
-  // stage record of a sample (floats): 8 dim-1 weights, CW dim-2 weights, ZN dim-0 weights, the
+  // stage record of a sample (floats): 8 dim-1 weights, CW dim-2 weights, R dim-0 weights, the
   // k-space values by component; padded so that 16-byte accesses of consecutive lanes spread over
   // all banks
-  static constexpr int XO = 8, ZO = XO + CW, YO = ZO + ZN;
+  static constexpr int XO = 8, ZN = R, ZO = XO + CW, YO = ZO + ZN;
   static constexpr int RS = (YO + YC * NB) % 8 == 4 ? YO + YC * NB : (YO + YC * NB + 8) / 8 * 8 - 4;
   static_assert(NBLK * RP >= SUB && (NARROW ? 3 : 7) + P <= CW && NBB <= 8, "blocks");
 };
 
 // Plane `pl` is final: store its slot (element E = pl mod 4) and clear it.
 template <class M, int E>
-__device__ __forceinline__ void retire_plane(const M& m, v4f (&acc)[M::NH][M::NBLK][M::NB], int pl, int lane,
+__device__ __forceinline__ void retire_plane(v4f (&acc)[M::NH][M::NBLK][M::NB], int pl, int lane,
                                              const SlotStore& out) {
   asm volatile("" : "+v"(lane));  // lane terms are formed here, not held in registers between calls
   const int i16 = lane & 15, q = lane >> 4;
-  const int comp = m.comp_of_group(q);
+  const int comp = M::comp_of_group(q);
   const int r = M::NARROW ? i16 >> 3 : 0, x = M::NARROW ? i16 & 7 : i16;
   const int loff = ((comp >> 1) * M::NB * M::SUBN + r * M::SUB + x) * 8 + (comp & 1) * 4;
-  const bool act = m.holds(q, pl);
+  const bool act = M::holds(q, pl);
   const bool lastrow = (M::NBLK - 1) * M::RP + r < M::SUB;  // rows of the last block
   const int l0 = act && x < M::SUB ? loff : kNoLane;
   const int l0e = lastrow ? l0 : kNoLane;
@@ -572,15 +569,14 @@ __device__ __forceinline__ void cells3_item(const float2* __restrict__ ksp, cons
                                             const float* __restrict__ wsort, const int* __restrict__ lbase,
                                             const int* __restrict__ perm, const Geom* __restrict__ geoms,
                                             const Item* __restrict__ items, const Geom& g, const Item& it, int iidx,
-                                            int c0, int nc, int slots, float2* __restrict__ scratch, float* rec,
+                                            int c0, int nc, float2* __restrict__ scratch, float* rec,
                                             int* list) {
   constexpr int P = M::P, NB = M::NB, SUB = M::SUB;
-  const M m(slots);
   int lane = threadIdx.x;
   asm volatile("" : "+v"(lane));  // keeps lane terms from being carried across the caller's loop
   const int i16 = lane & 15;
   const int kq = (lane >> 4) ^ 2;  // the group's sample in this lane's K slot (their order is free)
-  const int zl = m.slot(i16), comp = m.comp(i16);  // this lane's A row
+  const int zl = M::slot(i16), comp = M::comp(i16);  // this lane's A row
   const int br = M::NARROW ? i16 >> 3 : 0, bx = M::NARROW ? i16 & 7 : i16;  // B column: row, column in the block
   // byte offsets of this lane's operands from its group's first record
   const int off_w1 = (kq * M::RS + br * 4) * 4, off_w2 = (kq * M::RS + M::XO + bx) * 4;
@@ -616,7 +612,7 @@ __device__ __forceinline__ void cells3_item(const float2* __restrict__ ksp, cons
   clear_planes(dst2, last, SUB, nc, M::PP, M::SUBN, lane);
   int row = first;  // lowest plane not yet stored
   auto retire_to = [&](int to) {
-    for (; row < to; ++row) with_element(row, [&](auto E) { retire_plane<M, E.value>(m, acc, row, lane, out); });
+    for (; row < to; ++row) with_element(row, [&](auto E) { retire_plane<M, E.value>(acc, row, lane, out); });
   };
 
   bool any_odd = false;
@@ -680,7 +676,7 @@ __device__ __forceinline__ void cells3_item(const float2* __restrict__ ksp, cons
     } o;
     int g = 0, d = gr.at(0);  // the group whose operands are in `o`
     auto load_w0 = [&]() {  // this lane's ring slot holds patch plane zl - row (mod slots)
-      o.w0 = *(const float*)((const char*)rec + (d & 0xfff0) + off_w0 + m.slot(zl - row) * 4);
+      o.w0 = *(const float*)((const char*)rec + (d & 0xfff0) + off_w0 + M::slot(zl - row) * 4);
     };
     auto load = [&]() {
       const char* p = (const char*)rec + (d & 0xfff0);
@@ -739,8 +735,10 @@ __global__ __launch_bounds__(64) void grid_cells3d_kernel(const float2* __restri
                                                           const Geom* __restrict__ geoms,
                                                           const Item* __restrict__ items, int nitems, int nchunks,
                                                           float2* __restrict__ scratch) {
-  using M = Cells3<P, NB>;
-  __shared__ __attribute__((aligned(16))) float rec[kRows * M::RS];
+  constexpr int R = ring_slots(P);
+  using M = Cells3<P, NB, R>;
+  using W = Cells3<P, NB, 8>;
+  __shared__ __attribute__((aligned(16))) float rec[kRows * (P == 5 && W::RS > M::RS ? W::RS : M::RS)];
   __shared__ int list[kCh];
   int iidx, cc;
   item_of_block(blockIdx.x, nchunks, iidx, cc);
@@ -751,18 +749,22 @@ __global__ __launch_bounds__(64) void grid_cells3d_kernel(const float2* __restri
   const int c0 = cc * M::NC;
   if (c0 >= g.nbatch) return;
   const int nc = min(M::NC, g.nbatch - c0);
-  const int slots = M::DUAL && reaches_last_plane<3, P>(wsort, g, it) ? 8 : M::R0;
-  const int step = slots == M::R0 ? M::NC : NB;  // coils at a time
-  for (int c = 0; c < nc; c += step)
-    cells3_item<M>(ksp, dcf, wsort, lbase, perm, geoms, items, g, it, iidx, c0 + c, min(step, nc - c), slots, scratch, rec,
-               list);
+  if constexpr (P == 5) {
+    if (reaches_last_plane<3, P>(wsort, g, it)) {  // half the coils at a time
+      for (int c = 0; c < nc; c += W::NC)
+        cells3_item<W>(ksp, dcf, wsort, lbase, perm, geoms, items, g, it, iidx, c0 + c, min(W::NC, nc - c), scratch,
+                       rec, list);
+      return;
+    }
+  }
+  cells3_item<M>(ksp, dcf, wsort, lbase, perm, geoms, items, g, it, iidx, c0, nc, scratch, rec, list);
 }
 
 // ---- launch ---------------------------------------------------------------------------------
 
 template <int P, int T, int NB>
 void launch_rows2(const GridMfmaArgs& a) {
-  constexpr int NC = Rows2<P, T, NB>::NC;
+  constexpr int NC = NB * 8 / ring_slots(P);
   const int nch = (a.nbatch + NC - 1) / NC;
   grid_rows2d_kernel<P, T, NB><<<item_grid(a.nitems, nch), 64, 0, a.stream>>>(
       a.ksp, a.dcf, a.wsort, a.lbase, a.perm, a.geoms, a.items, a.nitems, nch, a.scratch);
@@ -770,19 +772,23 @@ void launch_rows2(const GridMfmaArgs& a) {
 
 template <int P, int NB>
 void launch_cells3(const GridMfmaArgs& a) {
-  constexpr int NC = Cells3<P, NB>::NC;
+  constexpr int NC = NB * 8 / ring_slots(P);
   const int nch = (a.nbatch + NC - 1) / NC;
   grid_cells3d_kernel<P, NB><<<item_grid(a.nitems, nch), 64, 0, a.stream>>>(
       a.ksp, a.dcf, a.wsort, a.lbase, a.perm, a.geoms, a.items, a.nitems, nch, a.scratch);
 }
 
 // Coils per wave. More of them share the staging and the control of a group, fewer leave more and
-// shorter waves, which is what these latency-bound launches need (131 k samples x 16 coils, 2D:
-// 2 / 4 / 8 / 16 coils per wave take 40 / 37 / 43 / 59 us at P = 5; at P = 7 1 / 2 / 4 / 8 coils
-// take 49 / 40 / 36 / 42 us). A single coil (or pair, with 4 slots) takes one block.
+// shorter waves, which is what these latency-bound launches need. 2D phase 1, us at 2 / 4 / 8 / 16
+// coils a wave, P = 5, and 1 / 2 / 4 / 8, P = 7:
+//   131 k spiral samples x 16    33 /  30 /  36 /  47      49 /  38 /  34 /  41
+//   131 k radial x 32            53 /  48 /  52 /  62      82 /  61 /  59 /  61
+//   2 M spiral x 32             498 / 382 / 382 / 406     868 / 590 / 491 / 481
+//   2 M radial x 32             777 / 829 / 822 / 870     874 / 780 / 814 / 825
+// A single coil (or pair, with 4 slots) takes one block.
 template <int P, int T>
 void launch_2d(const GridMfmaArgs& a) {
-  constexpr int per_block = 8 / Ring<P, 1>::R0;
+  constexpr int per_block = 8 / ring_slots(P);
   if (a.nbatch <= per_block) launch_rows2<P, T, 1>(a);
   else launch_rows2<P, T, 4 / per_block>(a);
 }
@@ -801,7 +807,7 @@ void launch_2d_t(int T, const GridMfmaArgs& a) {
 // 0.76 M x 7 at P = 7: 1 / 2 / 3 / 4 coils 0.34 / 0.38 / 0.42 / 0.45 ms.
 template <int P>
 void launch_3d(const GridMfmaArgs& a) {
-  if (P >= 6 || a.nbatch <= 8 / Ring<P, 1>::R0) launch_cells3<P, 1>(a);
+  if (P >= 6 || a.nbatch <= 8 / ring_slots(P)) launch_cells3<P, 1>(a);
   else launch_cells3<P, (P >= 6 ? 1 : 2)>(a);
 }
 
