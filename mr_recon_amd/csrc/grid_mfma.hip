@@ -36,10 +36,11 @@
 // and added to their patch one by one at the end (grid_odd_samples).
 //
 // What bounds it: latency in 2D (a wave's chain of chunks: 20 rows to store and ~16 groups per
-// chunk), the matrix pipe and the issue of the per-group control around it in 3D (36 % of the
-// matrix rate in the 3D 128^3 case, 2 waves per SIMD; skipping all but one of a group's products
-// takes 11 % off, skipping the gathers 20 %). Phase 1 before (2D: per-lane LDS read-modify-
-// writes; 3D: products per cell added to an LDS plane ring) and now, MI355X:
+// chunk; 131 k samples x 16 coils, P 5: matrix cores 12 % busy, LDS 10 %, and 44 % of the CU cycles
+// without a wave, since the launch ends on its longest items), in 3D the chains of its two waves
+// per SIMD (5.12 M x 32: matrix cores 41 % busy, LDS 15 %, 7.9 GB moved in 2.4 ms; skipping all
+// but one of a group's products takes 11 % off, skipping the gathers 20 %). Phase 1 before (2D:
+// per-lane LDS read-modify-writes; 3D: products per cell added to an LDS plane ring) and now, MI355X:
 //   3D 5.12 M samples x 32 coils, P 5   4.88 -> 2.30 ms     0.76 M x 7, P 7   1.00 -> 0.33 ms
 //   3D 1.5 M samples x 1, P 5            155 -> 110 us      2D 131 k x 16, P 5  80 -> 30 us
 //   2D 131 k samples x 16, P 7            94 -> 34 us       2D 4096 x 1, P 7    83 -> 15 us

@@ -20,7 +20,8 @@
 //  grid_partial  one wave accumulates its samples into LDS subgrids with plain
 //                (atomic-free) read-modify-writes, summing runs of samples in
 //                register windows, and stores each subgrid to a scratch slot with
-//                plain coalesced stores -- no global atomics.
+//                plain coalesced stores -- no global atomics. 2D with P <= 8 and 3D with
+//                P <= 7 run on the matrix cores instead (grid_mfma.hip).
 //  grid_reduce   one block per (output tile, coil) sums, in a fixed order, the
 //                scratch subgrids of every item whose subgrid covers the tile
 //                and writes the grid once. Device-scope float atomics run at a
@@ -418,7 +419,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, kIn
 #define MRA_GRID_CPL 1
 #endif
 #ifndef MRA_GRID_NSMAX
-#define MRA_GRID_NSMAX 12  // most coil slots per wave (12 over 8: batched 2D +14 %, same box)
+#define MRA_GRID_NSMAX 12  // most coil slots per wave (12 over 8: batched 2D +14 % while it ran here)
 #endif
 
 // LDS padding (row pitch of the last dim += E in 3D, coil-slot stride += SP), from a
